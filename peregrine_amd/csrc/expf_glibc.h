@@ -66,24 +66,26 @@ PHIP_HD inline double f64_from(uint64_t u) {
 
 }  // namespace phip_expf
 
-PHIP_HD inline float expf_glibc(float x) {
+// The method with the table behind t: t(i) = T[i], 0 <= i < 32. Branch-free:
+// x is clamped to [-104, 89], where the last rounding already gives 0 and
+// infinity, the results of everything beyond; NaN passes through.
+template <class Table>
+PHIP_HD inline float expf_glibc_t(float x, Table t) {
     using namespace phip_expf;
-    const uint32_t abstop = (f32_bits(x) >> 20) & 0x7ff;
-    if (abstop >= (f32_bits(88.0f) >> 20)) {   // |x| >= 88, inf or NaN
-        if (f32_bits(x) == f32_bits(-INFINITY)) return 0.0f;
-        if (abstop >= (f32_bits(INFINITY) >> 20)) return x + x;
-        if (x > 0x1.62e42ep6f) return INFINITY;   // above log(2^128)
-        if (x < -0x1.9fe368p6f) return 0.0f;      // below log(2^-150)
-    }
-    const double xd = (double)x;
+    const double xd = (double)fminf(fmaxf(x, -104.0f), 89.0f);
     double kd = fma(INV_LN2_N, xd, SHIFT);
     const uint64_t ki = f64_bits(kd);
     kd -= SHIFT;
     const double r = fma(INV_LN2_N, xd, -kd);
-    const double s = f64_from(T[ki % 32] + (ki << 47));
+    const double s = f64_from(t((uint32_t)ki % 32u) + (ki << 47));
     const double z = fma(C0, r, C1);
     const double r2 = r * r;
     double y = fma(C2, r, 1.0);
     y = fma(z, r2, y);
-    return (float)(y * s);
+    const float e = (float)(y * s);
+    return x != x ? x + x : e;
+}
+
+PHIP_HD inline float expf_glibc(float x) {
+    return expf_glibc_t(x, [](uint32_t i) { return phip_expf::T[i]; });
 }

@@ -325,6 +325,11 @@ __global__ __launch_bounds__((NW + 1) * 64) void gemv_kernel(DotArgs a, MatGeom 
     if (!chainer) load_round(0, wA, sA);
     __syncthreads();
 
+    ExpTab tab{};        // the chain wave's, loaded while the others stream
+    if (GATEUP && chainer) {   // uniform
+        tab = exp_tab();
+        exp_tab_pin(tab);
+    }
     float facc = 0.0f;   // chain accumulator (chain wave)
     int gsum = 0;        // EPI_GRP: open group's integer sum
     int isum = 0;        // EPI_ROW: exact integer sum
@@ -394,11 +399,11 @@ __global__ __launch_bounds__((NW + 1) * 64) void gemv_kernel(DotArgs a, MatGeom 
     }
     if constexpr (GATEUP) {
         const float u = __shfl(v, (lane & 31) + 32);
+        const float h = silu_mul(v, u, tab);   // lanes 32-63: unused
+        const float m = half_wave_max(fabsf(h));
         if (lane < 32) {
-            const float h = silu_mul(v, u);
             if (!(EPI == EPI_B32 && a.hq)) a.out[(size_t)r * a.out_stride + o] = h;   // else only hq / sh are read
             if (EPI == EPI_B32 && a.hq) {
-                const float m = warp_max(fabsf(h), 32);
                 float sc = __fdiv_rn(m, 127.0f);
                 if (sc < 1e-12f) sc = 1e-12f;
                 const float inv = __fdiv_rn(1.0f, sc);
@@ -605,11 +610,11 @@ __global__ __launch_bounds__(1024) void gemv_split_kernel(DotArgs a, MatGeom g, 
     }
     if constexpr (GATEUP) {
         const float uu = __shfl(v, (lane & 31) + 32);
+        const float h = silu_mul(v, uu, exp_tab());   // lanes 32-63: unused
+        const float m = half_wave_max(fabsf(h));
         if (lane < 32) {
-            const float h = silu_mul(v, uu);
             if (!(EPI == EPI_B32 && a.hq)) a.out[(size_t)r * a.out_stride + o] = h;   // else only hq / sh are read
             if (EPI == EPI_B32 && a.hq) {
-                const float m = warp_max(fabsf(h), 32);
                 float sc = __fdiv_rn(m, 127.0f);
                 if (sc < 1e-12f) sc = 1e-12f;
                 const float inv = __fdiv_rn(1.0f, sc);

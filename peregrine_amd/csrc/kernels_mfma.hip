@@ -245,16 +245,18 @@ __global__ __launch_bounds__(256) void mfma_kernel(DotArgs a, MatGeom g, const i
 
     if constexpr (GATEUP) {
         const int o = oc[0];
+        const ExpTab tab = exp_tab();
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
+            if (8 * (i >> 2) >= rend - r0) break;   // uniform: rows past the tile's end
             const int row = r0 + acc_row(i, lane);
-            const float h = silu_mul(v[0][i], v[1][i]);
+            const float h = silu_mul(v[0][i], v[1][i], tab);
             const bool ok = row < rend && o < ((g.O + 31) & ~31);
             // with the h quantisation fused, only hq / sh are read downstream
             if (ok && !(EPI == EPI_B32 && a.hq)) a.out[(size_t)row * a.out_stride + o] = h;
             if (EPI == EPI_B32 && a.hq) {
                 // one h row's 32 channels live in the 32 lanes of this half-wave
-                const float m = warp_max(fabsf(h), 32);
+                const float m = half_wave_max(fabsf(h));
                 float sc = __fdiv_rn(m, 127.0f);
                 if (sc < 1e-12f) sc = 1e-12f;
                 const float inv = __fdiv_rn(1.0f, sc);
@@ -330,6 +332,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GATEUP || !
     extern __shared__ __attribute__((aligned(16))) uint8_t lds_u8[];   // [NSTG][ST::BYTES], then sxl
 
     const int lane = threadIdx.x & 63, wave = wave_id();
+    ExpTab tab{};
+    if constexpr (GATEUP) tab = exp_tab();
     const int tile = blockIdx.y;
     if (tile >= a.plan.counts[1]) return;
     const int e = a.plan.mt_exp[tile], r0 = a.plan.mt_row0[tile], rend = a.plan.mt_rend[tile];
@@ -375,6 +379,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GATEUP || !
         if constexpr (EPI != EPI_ROW) lds_dma4(src_s + (size_t)grp_of(bc, g.gshift) * TILE_O, wv + ST::SW);
     };
 
+    if constexpr (GATEUP) exp_tab_pin(tab);
     // the tile's activation scales ([nb][32] in LDS) by LDS-DMA, all issued
     // at once: one copy per wave covers two blocks of the 32 rows. Nothing
     // waits on them before block 0's wait, which covers them (a wave's loads
@@ -526,13 +531,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GATEUP || !
         const int o = oc[0];
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
+            if (8 * (i >> 2) >= rend - r0) break;   // uniform: rows past the tile's end
             const int row = r0 + acc_row(i, lane);
-            const float h = silu_mul(v[0][i], v[1][i]);
+            const float h = silu_mul(v[0][i], v[1][i], tab);
             const bool ok = row < rend && o < ((g.O + 31) & ~31);
             // with the h quantisation fused, only hq / sh are read downstream
             if (ok && !(EPI == EPI_B32 && a.hq)) a.out[(size_t)row * a.out_stride + o] = h;
             if (EPI == EPI_B32 && a.hq) {
-                const float m = warp_max(fabsf(h), 32);
+                const float m = half_wave_max(fabsf(h));
                 float sc = __fdiv_rn(m, 127.0f);
                 if (sc < 1e-12f) sc = 1e-12f;
                 const float inv = __fdiv_rn(1.0f, sc);
@@ -603,6 +609,8 @@ __global__ __launch_bounds__(256) void mfma_sa_kernel(DotArgs a, MatGeom g) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds_u8[];   // [NSTG][ST::BYTES], then sxl
 
     const int lane = threadIdx.x & 63, wave = wave_id();
+    ExpTab tab{};
+    if constexpr (GATEUP) tab = exp_tab();
     // XO (dispatches that re-read each expert's weights over several M
     // tiles): workgroup L runs on XCD L mod 8, and each XCD takes a
     // contiguous run of the items in (expert, group of XO_G tiles, slab,
@@ -669,6 +677,7 @@ __global__ __launch_bounds__(256) void mfma_sa_kernel(DotArgs a, MatGeom g) {
             lds_dma4_s(voff_s, base_s + (size_t)grp_of(b, g.gshift) * 128, st + ST::S + wave * 256);
     };
 
+    if constexpr (GATEUP) exp_tab_pin(tab);
     // the tile's activation scales ([nb][32] in LDS), all issued at once:
     // one copy per wave covers two blocks of the 32 rows; block 0's wait
     // covers them (a wave's loads complete in order)
@@ -822,13 +831,14 @@ __global__ __launch_bounds__(256) void mfma_sa_kernel(DotArgs a, MatGeom g) {
         const int o = oc[0];
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
+            if (8 * (i >> 2) >= rend - r0) break;   // uniform: rows past the tile's end
             const int row = r0 + acc_row(i, lane);
-            const float h = silu_mul(v[0][i], v[1][i]);
+            const float h = silu_mul(v[0][i], v[1][i], tab);
             const bool ok = row < rend && o < ((g.O + 31) & ~31);
             // with the h quantisation fused, only hq / sh are read downstream
             if (ok && !(EPI == EPI_B32 && a.hq)) a.out[(size_t)row * a.out_stride + o] = h;
             if (EPI == EPI_B32 && a.hq) {
-                const float m = warp_max(fabsf(h), 32);
+                const float m = half_wave_max(fabsf(h));
                 float sc = __fdiv_rn(m, 127.0f);
                 if (sc < 1e-12f) sc = 1e-12f;
                 const float inv = __fdiv_rn(1.0f, sc);
