@@ -97,7 +97,8 @@ struct RowPlan {
     const int *mt_row0;    // [T] first row of the tile
     const int *mt_rend;    // [T] one past the last row of that expert
     const int *mt_first;   // [T] the first M tile of that expert (its tiles are consecutive)
-    const int *counts;     // [2] {R, T} as built on the device (or host)
+    const int *lead;       // [G] leading M tiles of each expert's groups of four (mfma_row_kernel)
+    const int *counts;     // [4] {R, T, -, G} as built on the device (or host)
     const ExpertDesc *row_desc;  // optional [R]: row r's descriptor, written by the router
 };
 
@@ -298,6 +299,7 @@ struct DotArgs {   // shared by the GEMV and MFMA arms
     int spin_limit;                                                     // GEMV: polls before a bounded wait gives up
     int *wait_failed;                                                   // GEMV: host-visible word, set to 1 when one does
     int w_reuse;                                                        // MFMA arm: M tiles re-read each expert's weights
+    int lead_bound;                                                     // > 0: per-row weights run mfma_row_kernel, G <= this
     RouteArgs route;                                                    // gate/up GEMV: logits != null -> fused router
     // down GEMV, one token (rows 0..n-1 in top-k order): the last workgroup
     // to finish an output tile also writes tail_out over that tile, the
@@ -357,11 +359,12 @@ void launch_gemv_down_combine(const DotArgs &a, const MatGeom &g, int act, int k
                               hipStream_t st);
 
 struct TableOut {
-    int *hdr;          // [4]: R, T, n_u, flags
+    int *hdr;          // [4]: R, T, n_u, G (0 without lead)
     int *uexp, *off;   // [E], [E+1]
     int *row_tok, *row_kk, *row_exp;  // [R]
     int *tok_rows, *tok_kk;           // [S*k]: each token's rows in union order (-1 pads), their top-k slot
     int *mt_exp, *mt_row0, *mt_rend, *mt_first;  // [Tmax]
+    int *lead;                        // optional [row_lead_bound]: the leading M tiles (RowPlan.lead)
 };
 void launch_synth_fill(void *dst, size_t n, int kind, float a, float b, uint64_t seed, hipStream_t st);
 // work: table_work_ints(S, k, E) ints of device scratch, fully rewritten by every call

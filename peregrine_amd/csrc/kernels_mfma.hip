@@ -18,6 +18,7 @@
 // int4 weights are unpacked in registers: 8 bytes (16 nibbles) per lane per
 // block -> 16 int8 values scaled by 16 (the scale tables carry the 1/16).
 #include <cstdlib>
+#include <type_traits>
 
 #include "common.h"
 #include "mfma_map.h"
@@ -876,6 +877,251 @@ static void launch_mfma_sa_h(const DotArgs &a, const MatGeom &g, int grid_tiles,
     launch_k(kern, grid, dim3(256), lds, st, a, g);
 }
 
+// ---------------------------------------------------------------------------
+// Per-row weights and activations (EPI_ROW), dispatches of about 24 or more
+// rows per expert (the rule and its measurements: row_groups in runtime.hip).
+// The int32 dots of a whole row of K accumulate inside the MFMA, so there is
+// no per-block f32 step, and what bounds the 32-row kernels here is everything
+// done once per 32 rows: fetching and unpacking the weights, a barrier and an
+// LDS round trip per two MFMAs. An item is therefore up to four M tiles (128
+// rows) of one expert times the slab of 8 subtiles: a wave unpacks its two
+// weight subtiles once for up to eight MFMAs, and a barrier covers two blocks.
+// Stages (two blocks each, RowStage::NST of them) are filled by scalar-base
+// LDS-DMA as in mfma_sa_kernel, the activations as 16-byte pieces (mfma_map.h).
+// Measured, 1777 tokens, top-8 of 160 experts with skewed popularity (14216
+// rows), D = 5120, I = 1536, int4: gate/up 506 -> 370 us, down 294 -> 225 us.
+// Without its copies it takes 238 / 142 us, without its MFMAs 316 / 170: the
+// weights of 222 items x 7.9 MB arrive at 5.5 TB/s. 161-165 VGPRs and 50 KB
+// of LDS: three workgroups per CU (two, with deeper stages: 406 / 247 us).
+// The items are spread evenly over the XCDs (mfma_map.h): in the contiguous
+// order of mfma_sa_kernel the XCDs that hold the rarely chosen experts get
+// most of them (772 / 469 us).
+// ---------------------------------------------------------------------------
+template <bool W4, int NM>   // NM: M tiles of the item
+struct RowStage {
+    static constexpr int CB = mmap::ROW_CB;
+    static constexpr int SUB = 32 * (W4 ? 16 : 32);    // one 32-column subtile of one block
+    static constexpr int A = 0;                        // [32 NM rows][64 B]
+    static constexpr int W = NM * 32 * 32 * CB;        // [CB][8 subtiles][SUB]
+    static constexpr int BYTES = W + CB * 8 * SUB;
+    static constexpr int FIT = (W4 ? 51200 : 81920) / BYTES;   // three (int8: two) workgroups per CU
+    static constexpr int NST = FIT < 5 ? FIT : 5;
+};
+
+template <bool W4, bool GATEUP, int NM>
+__device__ __forceinline__ void mfma_row_body(const DotArgs &a, const MatGeom &g, int slab, int e, int r0, int rend,
+                                              uint8_t *lds_u8, ExpTab tab) {
+    typedef RowStage<W4, NM> ST;
+    constexpr int CB = ST::CB, NST = ST::NST, BB = W4 ? 16 : 32;
+    constexpr int OPS_A = 2, OPS_W = CB * (W4 ? 1 : 2);   // copies per stage: a wave with rows of the item, every wave
+    const int lane = threadIdx.x & 63, wave = wave_id();
+    const int j = lane & 31, hh = lane >> 5;
+    const int nb = g.nb, nc = (nb + CB - 1) / CB;
+    const bool has_a = wave < NM;   // uniform
+    const uint32_t lds_addr = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds_u8);
+    auto act_row = [&](int r) { return a.act_identity ? r : a.plan.row_act[r]; };
+
+    // copy sources: uniform bases + per-lane offsets (rows past the expert's
+    // end repeat its last row, tiles past the tensor its last tile: never stored)
+    uint32_t voff_a[2], voff_a1[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int r = mmap::row_of(has_a ? wave : 0, i, lane), rr = min(r0 + r, rend - 1);
+        const uint32_t at = (uint32_t)act_row(rr) * (uint32_t)a.x_stride;
+        const int p = mmap::row_piece(r, lane & 3);
+        voff_a[i] = at + mmap::row_col(p, false);
+        voff_a1[i] = at + mmap::row_col(p, true);
+    }
+    const uint8_t *base_a = uniform_ptr(a.xq);
+    const int ntile = g.Op / TILE_O;
+    const uint8_t *base_w = uniform_ptr(a.desc[e].w[mmap::sa_mat(GATEUP, wave)]);
+    uint32_t voff_w, tile_w8[2] = {0, 0};
+    if constexpr (W4) {
+        voff_w = mmap::sa_voff_w4(GATEUP, slab, wave, lane, ntile, nb);
+    } else {
+        voff_w = mmap::row_voff_w8(lane);
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+            tile_w8[q] = __builtin_amdgcn_readfirstlane(mmap::sa_tile8(GATEUP, slab, wave, q, ntile, nb));
+    }
+    auto copy_stage = [&](int c, int stg) {
+        const uint32_t st = lds_addr + (uint32_t)(stg * ST::BYTES);
+        const int b0 = c * CB;
+        if (has_a) {
+            const bool one = b0 + 1 >= nb;   // uniform
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                lds_dma16_s(one ? voff_a1[i] : voff_a[i], base_a + (size_t)b0 * BLK,
+                            st + ST::A + (uint32_t)(wave * 2 + i) * 1024u);
+        }
+#pragma unroll
+        for (int q = 0; q < CB; ++q) {
+            const int b = min(b0 + q, nb - 1);
+            const uint8_t *wb = base_w + (size_t)b * ST::SUB;
+            const uint32_t dst = st + ST::W + (uint32_t)(q * 8 + wave * 2) * ST::SUB;
+            if constexpr (W4) {
+                lds_dma16_s(voff_w, wb, dst);
+            } else {
+#pragma unroll
+                for (int t = 0; t < 2; ++t) lds_dma16_s(voff_w, wb + tile_w8[t], dst + (uint32_t)t * ST::SUB);
+            }
+        }
+    };
+    // the epilogue's operands, loaded now: this lane's weight scales, and this
+    // thread's row's activation scale, shared through LDS after the loop
+    const int n0 = mmap::dma_n0(GATEUP, slab, wave);
+    int oc[2];
+    float sc[2];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+        oc[s] = GATEUP ? n0 + j : n0 + s * 32 + j;
+        const int o = min(oc[s], g.Op - 1);
+        sc[s] = gptr(a.desc[e].sc[GATEUP ? s : 2])[(size_t)(o / TILE_O) * g.ng * TILE_O + (o % TILE_O)];
+    }
+    const float sx_mine = a.sx[(size_t)act_row(min(r0 + ((int)threadIdx.x & 127), rend - 1)) * a.sx_stride];
+    if constexpr (GATEUP) exp_tab_pin(tab);
+#pragma unroll
+    for (int u = 0; u < NST - 1; ++u)
+        if (u < nc) copy_stage(u, u);
+
+    const int sub0 = GATEUP ? wave : 2 * wave, sub1 = GATEUP ? 4 + wave : 2 * wave + 1;
+    const uint32_t rd_w[2] = {(uint32_t)(ST::W + sub0 * ST::SUB), (uint32_t)(ST::W + sub1 * ST::SUB)};
+    const uint32_t rd_wl = W4 ? (uint32_t)(j * BB + hh * (BB / 2)) : (uint32_t)(hh * 512 + j * 16);
+    uint32_t rd_a[CB];   // row j of M tile 0; the swizzle repeats every 32 rows
+#pragma unroll
+    for (int q = 0; q < CB; ++q) rd_a[q] = mmap::row_rd(j, q, hh);
+
+    v16i acc[NM][2];
+#pragma unroll
+    for (int m = 0; m < NM; ++m) acc[m][0] = acc[m][1] = v16i{};
+    // the MFMAs of a stage's blocks [0, N)
+    auto mma_stage = [&](const uint8_t *st, auto n_const) {
+        constexpr int N = decltype(n_const)::value;
+        v4i A[N][NM];
+        uint2 w4[N][2];
+        v4i w8[N][2];
+#pragma unroll
+        for (int q = 0; q < N; ++q) {
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                const uint8_t *wp = st + rd_w[s] + rd_wl + q * 8 * ST::SUB;
+                if constexpr (W4) w4[q][s] = *(const uint2 *)wp;
+                else w8[q][s] = *(const v4i *)wp;
+            }
+#pragma unroll
+            for (int m = 0; m < NM; ++m) A[q][m] = *(const v4i *)(st + ST::A + m * 2048 + rd_a[q]);
+        }
+#pragma unroll
+        for (int q = 0; q < N; ++q) {
+            v4i B[2];
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                if constexpr (W4) {
+                    B[s][0] = i4_even16(w4[q][s].x);
+                    B[s][1] = i4_odd16(w4[q][s].x);
+                    B[s][2] = i4_even16(w4[q][s].y);
+                    B[s][3] = i4_odd16(w4[q][s].y);
+                } else {
+                    B[s] = w8[q][s];
+                }
+            }
+#pragma unroll
+            for (int m = 0; m < NM; ++m)
+#pragma unroll
+                for (int s = 0; s < 2; ++s)
+                    acc[m][s] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[q][m], B[s], acc[m][s], 0, 0, 0);
+        }
+    };
+    // stage c is complete in LDS, and every wave has read the stage before it:
+    // refill that one (its LDS reads are complete)
+    auto enter_stage = [&](int c, int prev) {
+        if (c + NST - 2 < nc) {   // uniform: only later stages' copies may be in flight
+            if (has_a) wait_vm<(NST - 2) * (OPS_A + OPS_W)>();
+            else wait_vm<(NST - 2) * OPS_W>();
+        } else {
+            wait_vm<0>();
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (c + NST - 1 < nc) copy_stage(c + NST - 1, prev);
+    };
+    int stg = 0, prev = NST - 1;
+    const int nfull = nb / CB;
+#pragma unroll 1
+    for (int c = 0; c < nfull; ++c) {
+        enter_stage(c, prev);
+        mma_stage(lds_u8 + stg * ST::BYTES, std::integral_constant<int, CB>());
+        prev = stg;
+        stg = stg + 1 == NST ? 0 : stg + 1;
+    }
+    if (nfull < nc) {   // odd nb: one block left
+        enter_stage(nfull, prev);
+        mma_stage(lds_u8 + stg * ST::BYTES, std::integral_constant<int, 1>());
+    }
+
+    // the item's activation scales through LDS (the stages are free once every wave is here)
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    float *sxl = (float *)lds_u8;
+    if (threadIdx.x < 128) sxl[threadIdx.x] = sx_mine;
+#pragma unroll
+    for (int s = 0; s < 2; ++s) sc[s] = W4 ? __fmul_rn(sc[s], 16.0f) : sc[s];   // W4 scale tables hold sw/16
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < NM; ++m) {
+#pragma unroll
+        for (int gq = 0; gq < 4; ++gq) {
+            if (r0 + 32 * m + 8 * gq >= rend) break;   // uniform: rows past the item's end
+            const float4 sq = *(const float4 *)(sxl + 32 * m + 8 * gq + 4 * hh);
+            const float sxr[4] = {sq.x, sq.y, sq.z, sq.w};
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const int i = 4 * gq + t, row = r0 + 32 * m + acc_row(i, lane);
+                float v[2];
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    const int D = W4 ? (acc[m][s][i] >> 4) : acc[m][s][i];
+                    v[s] = __fmul_rn(__fmul_rn((float)D, sc[s]), sxr[t]);
+                }
+                if constexpr (GATEUP) {
+                    const float h = silu_mul(v[0], v[1], tab);
+                    if (row < rend && oc[0] < ((g.O + 31) & ~31)) a.out[(size_t)row * a.out_stride + oc[0]] = h;
+                } else {
+#pragma unroll
+                    for (int s = 0; s < 2; ++s)
+                        if (row < rend && oc[s] < g.O) a.out[(size_t)row * a.out_stride + oc[s]] = v[s];
+                }
+            }
+        }
+    }
+}
+
+template <bool W4, bool GATEUP>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void mfma_row_kernel(DotArgs a, MatGeom g) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds_u8[];
+    ExpTab tab{};
+    if constexpr (GATEUP) tab = exp_tab();
+    int slab, i;
+    mmap::row_place((int)(blockIdx.x + gridDim.x * blockIdx.y), (int)gridDim.x, &slab, &i);
+    if (i >= a.plan.counts[3]) return;
+    const int tile = a.plan.lead[i];
+    const int e = a.plan.mt_exp[tile], r0 = a.plan.mt_row0[tile];
+    const int rend = min(a.plan.mt_rend[tile], r0 + mmap::ROW_TILES * MT_ROWS);
+    const int nm = (rend - r0 + MT_ROWS - 1) / MT_ROWS;   // uniform
+    if (nm == 4) mfma_row_body<W4, GATEUP, 4>(a, g, slab, e, r0, rend, lds_u8, tab);
+    else if (nm == 3) mfma_row_body<W4, GATEUP, 3>(a, g, slab, e, r0, rend, lds_u8, tab);
+    else if (nm == 2) mfma_row_body<W4, GATEUP, 2>(a, g, slab, e, r0, rend, lds_u8, tab);
+    else mfma_row_body<W4, GATEUP, 1>(a, g, slab, e, r0, rend, lds_u8, tab);
+}
+
+template <bool W4, bool GATEUP>
+static void launch_mfma_row(const DotArgs &a, const MatGeom &g, hipStream_t st) {
+    dim3 grid((unsigned)mmap::slab_count(GATEUP, g.O), (unsigned)mmap::row_grid(a.lead_bound));
+    const size_t lds = W4 ? 51200 : 81920;
+    auto kern = mfma_row_kernel<W4, GATEUP>;
+    static size_t opted[LDS_OPT_DEVICES];
+    lds_opt_in((const void *)kern, lds, opted);
+    launch_k(kern, grid, dim3(256), lds, st, a, g);
+}
+
 template <bool W4, int EPI, bool GATEUP, int PD>
 static void launch_mfma_p(const DotArgs &a, const MatGeom &g, int grid_tiles, hipStream_t st) {
     constexpr int NSUB = 2;
@@ -925,11 +1171,22 @@ static void launch_mfma_dma(const DotArgs &a, const MatGeom &g, int grid_tiles, 
     if constexpr (W4) {
         // weight-reuse dispatches in the XCD-aware expert-major order: config 4
         // gate/up fetch 3.69 -> 2.60 GB, down 1.50 -> 1.01 GB, step 1.5% faster
-        if (a.w_reuse) launch_mfma_sa_h<W4, EPI, GATEUP, PD, false, true>(a, g, grid_tiles, st);
-        else launch_mfma_sa_h<W4, EPI, GATEUP, PD, true>(a, g, grid_tiles, st);
+        // (per-row weights with as many rows run mfma_row_kernel)
+        if constexpr (EPI != EPI_ROW) {
+            if (a.w_reuse) {
+                launch_mfma_sa_h<W4, EPI, GATEUP, PD, false, true>(a, g, grid_tiles, st);
+                return;
+            }
+        }
+        launch_mfma_sa_h<W4, EPI, GATEUP, PD, true>(a, g, grid_tiles, st);
     } else {
-        if (a.w_reuse) launch_mfma_dma_h<W4, EPI, GATEUP, PD, false>(a, g, grid_tiles, st);
-        else launch_mfma_dma_h<W4, EPI, GATEUP, PD, true>(a, g, grid_tiles, st);
+        if constexpr (EPI != EPI_ROW) {
+            if (a.w_reuse) {
+                launch_mfma_dma_h<W4, EPI, GATEUP, PD, false>(a, g, grid_tiles, st);
+                return;
+            }
+        }
+        launch_mfma_dma_h<W4, EPI, GATEUP, PD, true>(a, g, grid_tiles, st);
     }
 }
 
@@ -945,6 +1202,12 @@ template <bool W4, int EPI, bool GATEUP>
 static void launch_mfma_t(const DotArgs &a, const MatGeom &g, int grid_tiles, hipStream_t st) {
     const int m = mfma_mode();
     if (!a.dots && m != 0) {
+        if constexpr (EPI == EPI_ROW) {
+            if (a.lead_bound > 0) {
+                launch_mfma_row<W4, GATEUP>(a, g, st);
+                return;
+            }
+        }
         if (mfma_dma_lds<W4, EPI, DMA_PD_SHALLOW>(g) <= 160 * 1024 / 3) {
             launch_mfma_dma<W4, EPI, GATEUP, DMA_PD_SHALLOW>(a, g, grid_tiles, st);
             return;

@@ -5,6 +5,7 @@
 #include <algorithm>
 
 #include "common.h"
+#include "mfma_map.h"
 #include "route.h"
 
 namespace phip {
@@ -503,22 +504,27 @@ __global__ __launch_bounds__(TBL_CHUNK) void table_count_kernel(const int *ids, 
 
 // Row offsets and M-tile offsets in union order, the M-tile list and the
 // header, from the experts in union order (uex[0..n_u)) and their counts.
-// base_out[e]: the expert's first row. ubuf: LDS for 2 * (n_u + 1) ints.
+// base_out[e]: the expert's first row. ubuf: LDS for 3 * (n_u + 1) ints. With
+// t.lead also the leading tiles of each expert's groups of four.
 // Workgroup-wide; ends synchronised.
 __device__ void table_offsets(int n_u, const int *uex, const int *cnt, int *base_out, const TableOut &t, int tmax,
                               int *scan_tmp, int *s_carry, int *ubuf) {
     const int tid = threadIdx.x, nth = blockDim.x;
-    int *offs = ubuf, *mts = ubuf + n_u + 1;   // per union rank: first row, first M tile
+    int *offs = ubuf, *mts = ubuf + n_u + 1, *lds = mts + n_u + 1;   // per union rank: first row, M tile, leading tile
+    constexpr int LT = mmap::ROW_TILES;
     for (int u0 = 0; u0 < n_u; u0 += nth) {
         const int u = u0 + tid;
         const int c = u < n_u ? cnt[uex[u]] : 0;
         const int off = block_exclusive_scan(c, scan_tmp) + (u0 ? s_carry[0] : 0);
         const int mt = block_exclusive_scan((c + MT_ROWS - 1) / MT_ROWS, scan_tmp) + (u0 ? s_carry[1] : 0);
+        const int nl = ((c + MT_ROWS - 1) / MT_ROWS + LT - 1) / LT;
+        const int ld = t.lead ? block_exclusive_scan(nl, scan_tmp) + (u0 ? s_carry[2] : 0) : 0;   // uniform
         if (u < n_u) {
             const int e = uex[u];
             base_out[e] = off;
             offs[u] = off;
             mts[u] = mt;
+            lds[u] = ld;
             t.uexp[u] = e;
             t.off[u] = off;
             if (u == n_u - 1) {
@@ -528,13 +534,14 @@ __device__ void table_offsets(int n_u, const int *uex, const int *cnt, int *base
                 t.hdr[0] = off + c;
                 t.hdr[1] = mt + (c + MT_ROWS - 1) / MT_ROWS;
                 t.hdr[2] = n_u;
-                t.hdr[3] = 0;
+                t.hdr[3] = t.lead ? ld + nl : 0;
             }
         }
         __syncthreads();
         if (tid == nth - 1) {
             s_carry[0] = off + c;
             s_carry[1] = mt + (c + MT_ROWS - 1) / MT_ROWS;
+            s_carry[2] = ld + nl;
         }
         __syncthreads();
     }
@@ -560,6 +567,7 @@ __device__ void table_offsets(int n_u, const int *uex, const int *cnt, int *base
         t.mt_row0[q] = offs[lo] + MT_ROWS * (q - mts[lo]);
         t.mt_rend[q] = offs[lo + 1];
         t.mt_first[q] = mts[lo];
+        if (t.lead && mmap::row_leads(q, mts[lo])) t.lead[lds[lo] + (q - mts[lo]) / LT] = q;
     }
     __syncthreads();
 }
@@ -574,7 +582,7 @@ __global__ __launch_bounds__(1024) void table_scan_kernel(int E, int G, const in
     __shared__ __attribute__((aligned(16))) int first[TBL_MAXE];
     __shared__ int cnt[TBL_MAXE], uex[TBL_MAXE];
     __shared__ int scan_tmp[32];
-    __shared__ int s_carry[2], s_nu;
+    __shared__ int s_carry[3], s_nu;
     const int tid = threadIdx.x, nth = blockDim.x;
     for (int e = tid; e < ((E + 3) & ~3); e += nth) {
         first[e] = INT_MAX;
@@ -726,9 +734,9 @@ __global__ __launch_bounds__(TBL_SMALL) void table_small_kernel(const int *ids, 
     __shared__ int sid[TBL_SMALL];
     __shared__ unsigned long long mask[TBL_MAXE * MW];
     __shared__ int first[TBL_MAXE], cnt[TBL_MAXE], uex[TBL_MAXE], rank[TBL_MAXE], base[TBL_MAXE];
-    __shared__ int ubuf[2 * (TBL_MAXE + 1)];
+    __shared__ int ubuf[3 * (TBL_MAXE + 1)];
     __shared__ int scan_tmp[32];
-    __shared__ int s_carry[2], s_nu;
+    __shared__ int s_carry[3], s_nu;
     const int tid = threadIdx.x;
     for (int e = tid; e < E; e += TBL_SMALL) {
         first[e] = INT_MAX;

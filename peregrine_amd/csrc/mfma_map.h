@@ -133,6 +133,39 @@ MMAP_HD int sx_row(int r0, int rend, int lane) {
 }
 MMAP_HD int sx_blk(int i, int lane, int nb) { return imin(2 * i + (lane >> 5), nb - 1); }
 
+// mfma_row_kernel (per-row weights and activations): an item is up to
+// ROW_TILES consecutive M tiles of one expert times a slab, a stage holds
+// ROW_CB blocks of K. Wave w copies the rows of the item's M tile w, 16 bytes
+// per lane: copy i covers rows 32w + 16i + lane/4, LDS slot lane%4 of the
+// row's 64 bytes. Slot s of row r holds 16-byte piece s ^ row_swz(r) (piece =
+// 2 * block-in-stage + K half), so that the 64-byte row stride of the operand
+// reads spreads over the LDS banks.
+constexpr int ROW_TILES = 4, ROW_CB = 2;
+// Each expert's tiles are led by its first, fifth, ...: item i of the list of
+// leading tiles times NS slabs. Workgroup L runs on XCD L mod 8, and leading
+// tile i's items all go to XCD i mod 8: its activations cross into one L2
+// only, and every XCD gets the same number of items (give or take NS). A
+// bijection of [0, NS * 8m) onto (slab, i < 8m): the grid's i are rounded up.
+MMAP_HD bool row_leads(int tile, int first) { return ((tile - first) & (ROW_TILES - 1)) == 0; }
+MMAP_HD int row_lead_bound(int R, int n_experts) { return R / (ROW_TILES * MT_ROWS) + n_experts; }
+MMAP_HD int row_grid(int leads) { return (leads + 7) & ~7; }
+MMAP_HD void row_place(int L, int NS, int *slab, int *i) {
+    const int seq = L >> 3;
+    *i = (seq / NS) * 8 + (L & 7);
+    *slab = seq % NS;
+}
+MMAP_HD int row_swz(int r) { return ((r >> 1) ^ (r >> 2)) & 3; }
+MMAP_HD int row_of(int wave, int i, int lane) { return 32 * wave + 16 * i + (lane >> 2); }
+MMAP_HD int row_piece(int r, int slot) { return slot ^ row_swz(r); }
+// source column of a piece, from the stage's first block; with only one block
+// left (odd nb) the second block's pieces repeat the first's (never used)
+MMAP_HD uint32_t row_col(int piece, bool one_block) { return (uint32_t)(one_block ? piece & 1 : piece) * 16u; }
+// LDS offset of row r's operand half hh of block q of the stage
+MMAP_HD uint32_t row_rd(int r, int q, int hh) { return (uint32_t)r * 64u + (uint32_t)((2 * q + hh) ^ row_swz(r)) * 16u; }
+// int8 weights: one copy per subtile and block, lane l takes column l%32, K
+// half l/32 (LDS order [half][column])
+MMAP_HD uint32_t row_voff_w8(int lane) { return (uint32_t)(lane & 31) * 32 + (uint32_t)(lane >> 5) * 16; }
+
 // Weight group of block b (per-row weights: gshift 30, every block in group 0).
 MMAP_HD int grp_of_blk(int b, int gshift) { return gshift >= 30 ? 0 : b >> gshift; }
 

@@ -16,6 +16,7 @@
 
 #include "../../include/peregrine_hip.h"
 #include "common.h"
+#include "mfma_map.h"
 
 using namespace phip;
 
@@ -691,6 +692,7 @@ struct DispatchOpts {
     int n_rows_fixed = -1;      // row count known on the host
     RouteArgs route{};          // one token: router + quant fused into the gate/up GEMV
     int w_reuse = 0;                    // about two or more M tiles per expert: weights stay cacheable
+    int lead_bound = 0;                 // > 0: the plan lists leading tiles, at most this many
     const float *combine_w = nullptr;   // one token: down + combine in one launch, weights [k]
     float *combine_out = nullptr;       //   and the layer output [D]
     const float *tail_w = nullptr;      // one token: the down GEMV's last workgroup per tile combines
@@ -769,6 +771,7 @@ void run_experts(Ctx *c, Prof &prof, const ExpertDesc *desc, const RowPlan &plan
     da.n_rows_fixed = opt.n_rows_fixed;
     da.route = opt.route;
     da.w_reuse = opt.w_reuse;
+    da.lead_bound = opt.lead_bound;
     da.spin_limit = g_spin_limit;
     da.wait_failed = c->wait_flag_dev;
     prof.mark(COLI_HIP_K_GATEUP);
@@ -809,6 +812,18 @@ void run_experts(Ctx *c, Prof &prof, const ExpertDesc *desc, const RowPlan &plan
     } else {
         launch_mfma_down(dd, gd, act, T_bound, c->stream);
     }
+}
+
+// Whether a dispatch of R rows over n experts runs mfma_row_kernel (per-row
+// weights and activations; items of up to 128 rows). It pays once experts
+// average about 24 rows: 160 experts, D = 5120, I = 1536, int4, layer time of
+// the 32-row kernel -> this one: 12.8 rows per expert (uniform routing) 387 ->
+// 414 us, 25.6 rows 475 -> 455, 51 rows 859 -> 538; skewed routing 25.6 rows
+// 563 -> 485, 89 rows 944 -> 745. With a short K its start and end weigh more
+// (K = 1000, 30 rows per expert: 71 -> 74 us), so there from 64 rows on.
+bool row_groups(const MatGeom &gg, const MatGeom &gd, int R, int n, int ga) {
+    if (epi_act(ga) != ACT_ROW || !(gg.per_row || gd.per_row)) return false;
+    return (long)R >= 64L * n || ((long)R >= 24L * n && gg.nb >= 64);
 }
 
 struct ReduceSpec {
@@ -975,7 +990,7 @@ int expert_group_impl(ColiHipTensor *const *gates, ColiHipTensor *const *ups, Co
     int T = 0;
     for (int i = 0; i < count; i++) T += (rows[i] + MT_ROWS - 1) / MT_ROWS;
     const int s_n = red ? red->s_n : 0;
-    const size_t n_int = (size_t)total /*row_exp*/ + 4 * (size_t)T + 2 + (red ? (size_t)(s_n + 1) + total : 0);
+    const size_t n_int = (size_t)total /*row_exp*/ + 5 * (size_t)T + 4 + (red ? (size_t)(s_n + 1) + total : 0);
     const size_t desc_b = round_up((size_t)count * sizeof(ExpertDesc), 16);
     // (a whole number of 16-byte words: the quantisation kernel stages it)
     const size_t meta_b = round_up(desc_b + n_int * 4 + (red ? (size_t)total * 4 : 0), 16);
@@ -1003,9 +1018,11 @@ int expert_group_impl(ColiHipTensor *const *gates, ColiHipTensor *const *ups, Co
     int *hi = (int *)(hm + desc_b);
     int *row_exp = hi, *mt_exp = row_exp + total, *mt_row0 = mt_exp + T, *mt_rend = mt_row0 + T;
     int *mt_first = mt_rend + T;
-    int *counts = mt_first + T;
-    int *rp = counts + 2, *ri = rp + (red ? s_n + 1 : 0);
+    int *lead = mt_first + T;
+    int *counts = lead + T;
+    int *rp = counts + 4, *ri = rp + (red ? s_n + 1 : 0);
     float *rwv = (float *)(ri + (red ? total : 0));
+    int G = 0;
     for (int i = 0, r = 0, t = 0; i < count; i++) {
         for (int q = 0; q < rows[i]; q++) row_exp[r + q] = i;
         const int t0 = t;
@@ -1014,11 +1031,14 @@ int expert_group_impl(ColiHipTensor *const *gates, ColiHipTensor *const *ups, Co
             mt_row0[t] = r + q;
             mt_rend[t] = r + rows[i];
             mt_first[t] = t0;
+            if (mmap::row_leads(t, t0)) lead[G++] = t;
         }
         r += rows[i];
     }
     counts[0] = total;
     counts[1] = T;
+    counts[2] = count;
+    counts[3] = G;
     if (red) {
         std::memcpy(rp, red->row_ptr, (size_t)(s_n + 1) * 4);
         std::memcpy(ri, red->row_idx, (size_t)total * 4);
@@ -1035,7 +1055,8 @@ int expert_group_impl(ColiHipTensor *const *gates, ColiHipTensor *const *ups, Co
     plan.mt_row0 = di + total + T;
     plan.mt_rend = di + total + 2 * T;
     plan.mt_first = di + total + 3 * T;
-    plan.counts = di + total + 4 * T;
+    plan.lead = di + total + 4 * T;
+    plan.counts = di + total + 5 * T;
     // No copy engine in the call: the staging buffers are mapped host
     // memory. The activation quantisation reads x across PCIe and also stages
     // the metadata into device memory (every later kernel reads it there); the
@@ -1046,6 +1067,7 @@ int expert_group_impl(ColiHipTensor *const *gates, ColiHipTensor *const *ups, Co
     DispatchOpts opt;
     if (arm == COLI_HIP_ARM_GEMV && !plan_split(c, gg, gd, total, epi_act(ga), false, &opt)) return 0;
     opt.w_reuse = total >= 2 * MT_ROWS * count;   // about two or more M tiles per expert
+    if (row_groups(gg, gd, total, count, ga)) opt.lead_bound = G;
     opt.meta_src = c->pin_meta.d;
     opt.meta_dst = dm;
     opt.meta_n16 = (int)(meta_b / 16);
@@ -1067,7 +1089,7 @@ int expert_group_impl(ColiHipTensor *const *gates, ColiHipTensor *const *ups, Co
         prof.mark(-1);
         if (phases) hipEventRecord(c->phase_ev[2], c->stream);
         if (red) {
-            const int *drp = plan.counts + 2, *dri = drp + s_n + 1;
+            const int *drp = plan.counts + 4, *dri = drp + s_n + 1;
             const float *drw = (const float *)(dri + total);
             prof.mark(COLI_HIP_K_COMBINE);
             launch_combine((float *)c->pin_y.d, s.y, drp, dri, drw, s_n, D, s.ys, c->stream);
@@ -1572,13 +1594,14 @@ int moe_forward_impl(const ColiHipExpertSet *set, const float *x_dev, int S, con
     if (!select_ctx(c)) return 0;
     const int E = set->count, R = S * k;
     const int tmax = (R + MT_ROWS - 1) / MT_ROWS + std::min(E, R);
+    const int lead_max = mmap::row_lead_bound(R, std::min(E, R));
     if (arm < 0) arm = forced_arm();
     if (arm < 0) arm = S == 1 ? COLI_HIP_ARM_GEMV : COLI_HIP_ARM_MFMA;
     const MatGeom &gg = set->gg, &gd = set->gd;
 
     // table layout in one buffer
     const size_t n_int =
-        4 + (size_t)E + (E + 1) + 3 * (size_t)R + 2 * (size_t)R + 4 * (size_t)tmax + table_work_ints(S, k, E);
+        4 + (size_t)E + (E + 1) + 3 * (size_t)R + 2 * (size_t)R + 4 * (size_t)tmax + (size_t)lead_max + table_work_ints(S, k, E);
     Scratch s{};
     int *p = nullptr;
     if (fixed_scratch) {
@@ -1627,6 +1650,8 @@ int moe_forward_impl(const ColiHipExpertSet *set, const float *x_dev, int S, con
     p += tmax;
     t.mt_first = p;
     p += tmax;
+    int *lead = p;
+    p += lead_max;
     int *tbl_work = p;
     c->tbl_view = t;
     c->tbl_E = E;
@@ -1636,6 +1661,10 @@ int moe_forward_impl(const ColiHipExpertSet *set, const float *x_dev, int S, con
     if (fixed_scratch) prof.on = false;   // profiling creates events: not on the no-allocation path
     DispatchOpts opt;
     opt.w_reuse = R >= 2 * MT_ROWS * E;   // about two or more M tiles per expert
+    if (row_groups(gg, gd, R, E, ga)) {
+        t.lead = lead;
+        opt.lead_bound = lead_max;
+    }
     const int act = epi_act(ga);
     // one token routes to k distinct experts in top-k order, which is also
     // batch-union order: row r is (token 0, slot r) and no table is needed
@@ -1701,6 +1730,7 @@ int moe_forward_impl(const ColiHipExpertSet *set, const float *x_dev, int S, con
         plan.mt_row0 = t.mt_row0;
         plan.mt_rend = t.mt_rend;
         plan.mt_first = t.mt_first;
+        plan.lead = t.lead;
         plan.counts = t.hdr;
     }
     run_experts(c, prof, set->desc_dev, plan, gg, gd, x_dev, S, false, R, tmax, ga, arm, s, opt);
