@@ -782,7 +782,9 @@ void run_experts(Ctx *c, Prof &prof, const ExpertDesc *desc, const RowPlan &plan
         launch_mfma_gateup(da, gg, act, T_bound, c->stream);
 
     if (act == ACT_ROW) {
-        QuantArgs qh{s.h, s.hs, R_bound, gd.K, gd.Kp, s.hq, s.hqs, s.sh, s.shs, ACT_ROW};
+        // h's columns up to Kp are written too (zero weights: zeros), so the
+        // rows are whole aligned groups whatever I is
+        QuantArgs qh{s.h, s.hs, R_bound, gd.Kp, gd.Kp, s.hq, s.hqs, s.sh, s.shs, ACT_ROW};
         prof.mark(COLI_HIP_K_QUANT_H);
         launch_quant_rows(qh, c->stream);
     }
