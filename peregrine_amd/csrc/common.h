@@ -264,12 +264,24 @@ inline void launch_k(K kern, dim3 grid, dim3 block, size_t lds, hipStream_t st, 
     }
 }
 
+struct TableOut {
+    int *hdr;          // [4]: R, T, n_u, G (0 without lead)
+    int *uexp, *off;   // [E], [E+1]
+    int *row_tok, *row_kk, *row_exp;  // [R]
+    int *tok_rows, *tok_kk;           // [S*k]: each token's rows in union order (-1 pads), their top-k slot
+    int *mt_exp, *mt_row0, *mt_rend, *mt_first;  // [Tmax]
+    int *lead;                        // optional [row_lead_bound]: the leading M tiles (RowPlan.lead)
+};
+
 struct QuantArgs {
     const float *x; int x_stride; int rows; int K; int Kp;
     int8_t *q; int q_stride; float *s; int s_stride; int mode;
     // optional: the workgroups also copy n16 16-byte words src -> dst (a
     // host-buffer call's metadata, staged from mapped host memory)
     const uint4 *copy_src; uint4 *copy_dst; int copy_n16;
+    // optional: one workgroup more builds the expert table of one token's k
+    // ids (k <= 16), so that it needs no launch of its own
+    const int *one_ids; int one_k, one_E; TableOut one_t;
 };
 void launch_quant_rows(const QuantArgs &a, hipStream_t st);
 
@@ -307,7 +319,12 @@ struct DotArgs {   // shared by the GEMV and MFMA arms
     // tail_ctr holds one arrival counter per tile, zero between dispatches
     float *tail_out;
     const float *tail_w;
+    const int *tail_kk;   // optional: row r's weight is tail_w[tail_kk[r]] (rows of a table), else tail_w[r]
     int *tail_ctr;
+    // down GEMV, per-row weights and activations: the f32 rows of h, which the
+    // workgroups quantise themselves (xq / sx are not read); null: xq / sx
+    const float *hf;
+    int hf_stride;
     // split-K GEMV (split > 1): each (row, output tile) unit's K blocks are
     // spread over `split` workgroups of split_kb blocks each; they park their
     // exact block dots and f32 factors in part_d / part_f and count in on
@@ -353,19 +370,13 @@ void launch_route_quant(const float *logits, int S, int E, int k, int *ids, floa
 constexpr int GEMV_SPIN_LIMIT = 1 << 22;
 // LDS bytes one workgroup may use (device attribute), set at init.
 void set_lds_limit(int bytes);
+// per-row weights: the down GEMV quantises h itself (DotArgs.hf)
+bool gemv_row_ok(const MatGeom &gd);
 // one token: down GEMV + router-weighted combine in one launch (k rows in top-k order)
 bool gemv_down_combine_ok(const MatGeom &g, int k);
 void launch_gemv_down_combine(const DotArgs &a, const MatGeom &g, int act, int k, const float *w, float *out,
                               hipStream_t st);
 
-struct TableOut {
-    int *hdr;          // [4]: R, T, n_u, G (0 without lead)
-    int *uexp, *off;   // [E], [E+1]
-    int *row_tok, *row_kk, *row_exp;  // [R]
-    int *tok_rows, *tok_kk;           // [S*k]: each token's rows in union order (-1 pads), their top-k slot
-    int *mt_exp, *mt_row0, *mt_rend, *mt_first;  // [Tmax]
-    int *lead;                        // optional [row_lead_bound]: the leading M tiles (RowPlan.lead)
-};
 void launch_synth_fill(void *dst, size_t n, int kind, float a, float b, uint64_t seed, hipStream_t st);
 // work: table_work_ints(S, k, E) ints of device scratch, fully rewritten by every call
 size_t table_work_ints(int S, int k, int E);

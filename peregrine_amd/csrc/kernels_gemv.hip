@@ -97,7 +97,13 @@ __device__ __forceinline__ void spin_until_geq(int *ctr, int target, int limit, 
 // (stores and loads with the SC1 cache policy: written through to, and read
 // from, the device coherence point), not on a language-level release/acquire
 // pair, whose whole-L2 write-back and invalidate is what the scheme avoids.
-__device__ __forceinline__ void tail_combine(const DotArgs &a, int O, int nrows, int o, int tile) {
+// wl: the rows' weights, row j's in lane j (tail_weight, loaded early).
+__device__ __forceinline__ float tail_weight(const DotArgs &a, int nrows) {
+    const int lane = threadIdx.x & 63;
+    if (!a.tail_out || lane >= nrows) return 0.0f;
+    return a.tail_w[a.tail_kk ? a.tail_kk[lane] : lane];
+}
+__device__ __forceinline__ void tail_combine(const DotArgs &a, int O, int nrows, int o, int tile, float wl) {
     const int lane = threadIdx.x & 63;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     int old = 0;
@@ -106,19 +112,26 @@ __device__ __forceinline__ void tail_combine(const DotArgs &a, int O, int nrows,
     if (old != nrows - 1) return;   // uniform
     asm volatile("" ::: "memory");
     const int oc = o < O ? o : O - 1;
-    float yv[GEMV_TAIL_MAXK], wv[GEMV_TAIL_MAXK];
+    float yv[GEMV_TAIL_MAXK];
 #pragma unroll
     for (int j = 0; j < GEMV_TAIL_MAXK; ++j) {   // every load issued before the sum
         const int jj = j < nrows ? j : 0;
         yv[j] = __hip_atomic_load(&a.out[(size_t)jj * a.out_stride + oc], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        wv[j] = a.tail_w[jj];
     }
     float acc = 0.0f;
 #pragma unroll
     for (int j = 0; j < GEMV_TAIL_MAXK; ++j)
-        if (j < nrows) acc = __fadd_rn(acc, __fmul_rn(wv[j], yv[j]));
+        if (j < nrows)
+            acc = __fadd_rn(acc, __fmul_rn(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(wl), j)), yv[j]));
     if (o < O) a.tail_out[o] = acc;
     if (lane == 0) __hip_atomic_store(&a.tail_ctr[tile], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// A tail combine with no row at all (every id out of range): the output is
+// zeros, written by the workgroups of row 0.
+__device__ __forceinline__ void tail_no_rows(const DotArgs &a, int O, int nrows, int tile) {
+    const int o = tile * 64 + (int)threadIdx.x;
+    if (a.tail_out && nrows == 0 && blockIdx.y == 0 && threadIdx.x < 64 && o < O) a.tail_out[o] = 0.0f;
 }
 
 // NW streaming waves plus one chain wave. K is walked in rounds of NW*CH
@@ -155,7 +168,10 @@ __global__ __launch_bounds__((NW + 1) * 64) void gemv_kernel(DotArgs a, MatGeom 
     const bool chainer = wave == NW;
     const int r = blockIdx.y;
     const int nrows = a.n_rows_fixed >= 0 ? a.n_rows_fixed : a.plan.counts[0];
-    if (r >= nrows) return;  // uniform: fewer rows than the grid bound
+    if (r >= nrows) {  // uniform: fewer rows than the grid bound
+        if constexpr (!GATEUP) tail_no_rows(a, g.O, nrows, (int)blockIdx.x);
+        return;
+    }
 
     const ExpertDesc *dsc;
     if constexpr (ROUTE) {
@@ -326,9 +342,14 @@ __global__ __launch_bounds__((NW + 1) * 64) void gemv_kernel(DotArgs a, MatGeom 
     __syncthreads();
 
     ExpTab tab{};        // the chain wave's, loaded while the others stream
+    float wl = 0.0f;
     if (GATEUP && chainer) {   // uniform
         tab = exp_tab();
         exp_tab_pin(tab);
+    }
+    if (!GATEUP && chainer) {
+        wl = tail_weight(a, nrows);
+        asm volatile("" : "+v"(wl));   // loaded here, not at the tail
     }
     float facc = 0.0f;   // chain accumulator (chain wave)
     int gsum = 0;        // EPI_GRP: open group's integer sum
@@ -416,7 +437,7 @@ __global__ __launch_bounds__((NW + 1) * 64) void gemv_kernel(DotArgs a, MatGeom 
             if (o < g.O) a.out[(size_t)r * a.out_stride + o] = v;
         } else {
             if (o < g.O) __hip_atomic_store(&a.out[(size_t)r * a.out_stride + o], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            tail_combine(a, g.O, nrows, o, (int)blockIdx.x);
+            tail_combine(a, g.O, nrows, o, (int)blockIdx.x, wl);
         }
     }
 }
@@ -468,7 +489,12 @@ __global__ __launch_bounds__(1024) void gemv_split_kernel(DotArgs a, MatGeom g, 
     const int S = a.split, kb = a.split_kb, nb = g.nb;
     const int u = (int)blockIdx.x / S, s = (int)blockIdx.x - u * S, r = blockIdx.y;
     const int nrows = a.n_rows_fixed >= 0 ? a.n_rows_fixed : a.plan.counts[0];
-    if (r >= nrows) return;   // uniform: fewer rows than the grid bound
+    if (r >= nrows) {   // uniform: fewer rows than the grid bound
+        if constexpr (!GATEUP) {
+            if (s == 0) tail_no_rows(a, g.O, nrows, u);
+        }
+        return;
+    }
     const int ntx = (int)gridDim.x / S;
     const size_t unit = (size_t)r * ntx + u;
     const int nbd = W4 ? (nb + 1) >> 1 : nb;   // dwords of parked dots per lane
@@ -627,9 +653,163 @@ __global__ __launch_bounds__(1024) void gemv_split_kernel(DotArgs a, MatGeom g, 
             if (o < g.O) a.out[(size_t)r * a.out_stride + o] = v;
         } else {
             if (o < g.O) __hip_atomic_store(&a.out[(size_t)r * a.out_stride + o], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            tail_combine(a, g.O, nrows, o, u);
+            tail_combine(a, g.O, nrows, o, u, tail_weight(a, nrows));
         }
     }
+}
+
+// ---------------------------------------------------------------------------
+// Per-row weights and activations (EPI_ROW): integer sums have no order, so
+// every wave streams its own blocks, sums its dots in a register, and the
+// waves' sums meet once in LDS: no ring, no chain wave. A wave's CH block
+// loads of a round are one batch; blocks b = (c * NW + wave) * CH + [0, CH).
+//
+// Down (a.hf): the workgroup quantises its row of h itself (quant.rs:14-33,
+// quant_rows_kernel's arithmetic) into LDS, every workgroup of the row the
+// same codes. The loads of h are issued before the weights', so the
+// quantisation runs while the weights arrive; it takes a launch off the path.
+// Waves read their blocks of codes from LDS as broadcasts.
+//
+// What bounds it at one token, top-8, D = 5120, I = 1536, int4 (63 + 31 MB):
+// the ramp and drain of 384 / 640 workgroups that are all resident at once,
+// 14.2 us gate/up (14.4 with the ring) and 8.4-9.3 us down with the
+// quantisation (8.9 without, plus 3.4 us for its launch). 5 x 16 waves x blocks
+// for gate/up takes 20 us; 8 x 10, 11 x 5, 16 x 10 and down 6 x 8, 8 x 6, 3 x 8,
+// 2 x 12 measure within 1 us of 10 x 8 and 4 x 12.
+// ---------------------------------------------------------------------------
+constexpr int GEMV_ROW_MAXK = 4096;   // of the down projection: codes in LDS, 4 * HPER floats of h per thread
+constexpr int GEMV_ROW_MAXSUM = 65536;   // 16 x 8 x 127 x K stays below 2^31
+template <bool W4, bool GATEUP, int NW, int CH>
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(GATEUP ? 1 : 4))) void gemv_row_kernel(DotArgs a, MatGeom g) {
+    constexpr int BB = W4 ? 16 : 32, NT = NW * 64;
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    __shared__ int red[NW][64];
+    __shared__ float mred[NW];
+    extern __shared__ __attribute__((aligned(16))) int8_t hl[];   // down: the row's codes [Kp]
+    const int lane = threadIdx.x & 63, wave = wave_id();
+    const int r = blockIdx.y;
+    const int nrows = a.n_rows_fixed >= 0 ? a.n_rows_fixed : a.plan.counts[0];
+    if (r >= nrows) {  // uniform: fewer rows than the grid bound
+        if constexpr (!GATEUP) tail_no_rows(a, g.O, nrows, (int)blockIdx.x);
+        return;
+    }
+    ExpTab tab{};
+    if constexpr (GATEUP) tab = exp_tab();
+    float wl = 0.0f;
+    if (!GATEUP && wave == 0) wl = tail_weight(a, nrows);
+    constexpr int HPER = GATEUP ? 1 : (GEMV_ROW_MAXK / 4 + NT - 1) / NT;
+    f4 hv[HPER];
+    const int nh = g.Kp >> 2;
+    if constexpr (!GATEUP) {
+        const auto *hp = (const __attribute__((address_space(1))) f4 *)gptr(a.hf + (size_t)r * a.hf_stride);
+#pragma unroll
+        for (int i = 0; i < HPER; ++i) {
+            hv[i] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+            if ((int)threadIdx.x + i * NT < nh) hv[i] = hp[threadIdx.x + i * NT];
+        }
+    }
+    const ExpertDesc *dsc = a.plan.row_desc ? &a.plan.row_desc[r] : &a.desc[a.plan.row_exp[r]];
+    const int half = lane >> 5, ol = lane & 31;
+    const int o = GATEUP ? (int)blockIdx.x * 32 + ol : (int)blockIdx.x * 64 + lane;
+    const int mat = GATEUP ? half : 2;
+    const int tile = GATEUP ? (int)blockIdx.x : 2 * (int)blockIdx.x + half;
+    const auto *wp = gptr(dsc->w[mat] + ((size_t)tile * g.nb * TILE_O + ol) * BB);
+    const float sw = gptr(dsc->sc[mat])[(size_t)tile * TILE_O + ol];
+    const int arow = a.act_identity ? r : (a.act_zero ? 0 : a.plan.row_act[r]);
+    const CInt *xs = (const CInt *)(a.xq + (size_t)arow * a.x_stride);
+    const int nb = g.nb;
+    WBlk<W4> wv[CH];
+    auto load_w = [&](int b0) {
+#pragma unroll
+        for (int j = 0; j < CH; ++j)
+            wv[j] = load_wblk<W4>((const uint8_t *)(wp + (size_t)min(b0 + j, nb - 1) * (TILE_O * BB)));
+    };
+    load_w(wave * CH);
+    float sx;
+    if constexpr (GATEUP) {
+        sx = ((const CFloat *)(a.sx + (size_t)arow * a.sx_stride))[0];
+    } else {
+        float m = 0.0f;
+#pragma unroll
+        for (int i = 0; i < HPER; ++i)
+            m = fmaxf(fmaxf(m, fmaxf(fabsf(hv[i].x), fabsf(hv[i].y))), fmaxf(fabsf(hv[i].z), fabsf(hv[i].w)));
+        m = warp_max(m, 64);
+        if (lane == 0) mred[wave] = m;
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < NW; ++w) m = fmaxf(m, mred[w]);
+        sx = __fdiv_rn(m, 127.0f);
+        if (sx < 1e-12f) sx = 1e-12f;
+        const float inv = __fdiv_rn(1.0f, sx);
+        auto code = [&](float f) { return (uint32_t)(uint8_t)(int8_t)(int)rintf(__fmul_rn(f, inv)); };
+#pragma unroll
+        for (int i = 0; i < HPER; ++i) {
+            const int f = (int)threadIdx.x + i * NT;
+            if (f < nh) {   // elements 4f..4f+3 in the device byte order: two pairs
+                uint16_t *d = (uint16_t *)(hl + (f >> 1) * 8 + (f & 1) * 2);
+                d[0] = (uint16_t)(code(hv[i].x) | code(hv[i].z) << 8);
+                d[2] = (uint16_t)(code(hv[i].y) | code(hv[i].w) << 8);
+            }
+        }
+        __syncthreads();
+    }
+    int isum = 0;
+#pragma unroll 1
+    for (int b0 = wave * CH;;) {
+        if constexpr (GATEUP) {
+            int xr[CH][8];   // uniform: SGPRs
+#pragma unroll
+            for (int j = 0; j < CH; ++j)
+#pragma unroll
+                for (int q = 0; q < 8; ++q) xr[j][q] = xs[min(b0 + j, nb - 1) * (BLK / 4) + q];
+#pragma unroll
+            for (int j = 0; j < CH; ++j) {
+                const int d = dot_wblk<W4>(wv[j], xr[j]);
+                isum += b0 + j < nb ? d : 0;   // uniform condition
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < CH; ++j) {
+                const int4 *xl = (const int4 *)(hl + min(b0 + j, nb - 1) * BLK);
+                const int4 q0 = xl[0], q1 = xl[1];
+                const int xb[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
+                const int d = dot_wblk<W4>(wv[j], xb);
+                isum += b0 + j < nb ? d : 0;
+                if (j & 1) asm volatile("" : "+v"(isum)::"memory");   // two blocks' codes at a time, not all in registers
+            }
+        }
+        b0 += NW * CH;
+        if (b0 >= nb) break;   // uniform
+        load_w(b0);
+    }
+    red[wave][lane] = isum;
+    __syncthreads();
+    if (wave != 0) return;
+    int D = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) D += red[w][lane];
+    if (W4) D >>= 4;   // unpacked int4 operands carry a factor 16
+    const float sc = W4 ? __fmul_rn(sw, 16.0f) : sw;
+    const float v = __fmul_rn(__fmul_rn((float)D, sc), sx);
+    if constexpr (GATEUP) {
+        const float u = __shfl(v, (lane & 31) + 32);
+        const float h = silu_mul(v, u, tab);   // lanes 32-63: unused
+        if (lane < 32) a.out[(size_t)r * a.out_stride + o] = h;
+    } else if (!a.tail_out) {
+        if (o < g.O) a.out[(size_t)r * a.out_stride + o] = v;
+    } else {
+        if (o < g.O) __hip_atomic_store(&a.out[(size_t)r * a.out_stride + o], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        tail_combine(a, g.O, nrows, o, (int)blockIdx.x, wl);
+    }
+}
+
+bool gemv_row_ok(const MatGeom &gd) { return gd.per_row && gd.Kp <= GEMV_ROW_MAXK; }
+
+template <bool W4, bool GATEUP>
+static void launch_gemv_row(const DotArgs &a, const MatGeom &g, int grid_rows, hipStream_t st) {
+    constexpr int NW = GATEUP ? (W4 ? 10 : 8) : 4, CH = GATEUP ? (W4 ? 8 : 5) : (W4 ? 12 : 6);
+    const dim3 grid(GATEUP ? (unsigned)((g.O + 31) / 32) : (unsigned)((g.O + 63) / 64), (unsigned)grid_rows);
+    launch_k((gemv_row_kernel<W4, GATEUP, NW, CH>), grid, dim3(NW * 64), GATEUP ? 0 : (size_t)g.Kp, st, a, g);
 }
 
 GemvSplit plan_gemv_split(const MatGeom &g, bool gateup, int rows, int act, int target_wgs) {
@@ -844,6 +1024,12 @@ static void launch_gemv_t(const DotArgs &a, const MatGeom &g, int grid_rows, hip
         if (ch == 4) launch_k((gemv_split_kernel<W4, EPI, GATEUP, 4>), grid, block, 0, st, a, g, a.xq, a.sx);
         else launch_k((gemv_split_kernel<W4, EPI, GATEUP, 2>), grid, block, 0, st, a, g, a.xq, a.sx);
         return;
+    }
+    if constexpr (EPI == EPI_ROW) {
+        if (!a.dots && !a.route.logits && (GATEUP ? g.Kp <= GEMV_ROW_MAXSUM : a.hf != nullptr)) {
+            launch_gemv_row<W4, GATEUP>(a, g, grid_rows, st);
+            return;
+        }
     }
     if constexpr (GATEUP) {
         if (a.route.logits) {

@@ -25,6 +25,58 @@ __device__ __forceinline__ void quant_side_copy(const QuantArgs &a) {
         a.copy_dst[i] = a.copy_src[i];
 }
 
+// The expert table of one token, by one wavefront (lane j: slot j): what
+// table_small_kernel writes for S = 1. Ids out of range are skipped, a
+// repeated expert's rows keep slot order. As one more workgroup of the
+// quantisation it is off the path (table_small_kernel: 5.6 us of 43 there).
+__device__ __forceinline__ void table_one(const int *ids, int k, int E, const TableOut &t) {
+    const int j = threadIdx.x & 63;
+    int e = j < k ? ids[j] : -1;
+    if (e < 0 || e >= E) e = -1;
+    int first = j;   // the expert's first slot
+    for (int i = k - 1; i >= 0; i--)
+        if (__builtin_amdgcn_readlane(e, i) == e) first = i;
+    const bool ok = e >= 0;
+    int row = 0, rank = 0, cnt = 0, nv = 0, nu = 0, inv_before = 0;
+    for (int i = 0; i < k; i++) {
+        const int ei = __builtin_amdgcn_readlane(e, i), fi = __builtin_amdgcn_readlane(first, i);
+        if (ei < 0) {
+            inv_before += i < j;
+            continue;
+        }
+        nv++;
+        nu += fi == i;
+        rank += fi == i && fi < first;
+        row += fi < first || (fi == first && i < j);
+        cnt += ei == e;
+    }
+    if (j < k) {
+        const int at = ok ? row : nv + inv_before;
+        t.tok_rows[at] = ok ? row : -1;
+        t.tok_kk[at] = ok ? j : 0;
+        if (ok) {
+            t.row_tok[row] = 0;
+            t.row_kk[row] = j;
+            t.row_exp[row] = e;
+            if (first == j) {   // at most 16 rows: one M tile per expert
+                t.uexp[rank] = e;
+                t.off[rank] = row;
+                t.mt_exp[rank] = e;
+                t.mt_row0[rank] = row;
+                t.mt_rend[rank] = row + cnt;
+                t.mt_first[rank] = rank;
+            }
+        }
+    }
+    if (j == 0) {
+        t.off[nu] = nv;
+        t.hdr[0] = nv;
+        t.hdr[1] = nu;
+        t.hdr[2] = nu;
+        t.hdr[3] = 0;
+    }
+}
+
 // ACT_ROW, rows of 16-byte aligned groups of 4 elements: WPR waves per row
 // (four waves per workgroup). All of a row's loads are in flight at once and
 // it is quantised from registers (beyond 64 * WPR * PER groups it is read
@@ -37,6 +89,10 @@ __device__ __forceinline__ void quant_side_copy(const QuantArgs &a) {
 // faster ones (192 rows of 5120: 73 us against 94).
 template <int WPR>
 __global__ __launch_bounds__(256) void quant_rows_vec_kernel(QuantArgs a) {
+    if (a.one_ids && blockIdx.x == gridDim.x - 1) {
+        if (threadIdx.x < 64) table_one(a.one_ids, a.one_k, a.one_E, a.one_t);
+        return;
+    }
     typedef float f4 __attribute__((ext_vector_type(4)));
     constexpr int PER = 8, NT = 64 * WPR;
     const int tid = threadIdx.x, t = tid & (NT - 1);
@@ -90,6 +146,10 @@ __global__ __launch_bounds__(256) void quant_rows_vec_kernel(QuantArgs a) {
 }
 
 __global__ __launch_bounds__(1024) void quant_rows_kernel(QuantArgs a) {
+    if (a.one_ids && blockIdx.x == gridDim.x - 1) {
+        if (threadIdx.x < 64) table_one(a.one_ids, a.one_k, a.one_E, a.one_t);
+        return;
+    }
     quant_side_copy(a);
     // ACT_ROW, any row: one workgroup per row; every thread loads its elements
     // in one round, then a block reduction gives the row's amax.
@@ -128,6 +188,10 @@ __global__ __launch_bounds__(1024) void quant_rows_kernel(QuantArgs a) {
 }
 
 __global__ __launch_bounds__(256) void quant_blocks_kernel(QuantArgs a) {
+    if (a.one_ids && blockIdx.y == gridDim.y - 1) {
+        if (blockIdx.x == 0 && threadIdx.x < 64) table_one(a.one_ids, a.one_k, a.one_E, a.one_t);
+        return;
+    }
     quant_side_copy(a);
     // ACT_B32: 8 elements per thread, a workgroup covers 64 blocks of one row
     const int row = blockIdx.y, nbk = a.Kp / BLK;
@@ -141,15 +205,17 @@ void launch_quant_rows(const QuantArgs &a, hipStream_t st) {
     // 16-byte loads need rows that start and end on 4 aligned elements; a
     // staging copy marks a host-buffer call, whose rows are in host memory
     const bool vec = a.copy_n16 == 0 && a.K % 4 == 0 && a.x_stride % 4 == 0 && ((uintptr_t)a.x & 15) == 0;
+    const unsigned more = a.one_ids ? 1 : 0;   // the workgroup that builds one token's table
     if (a.mode == ACT_ROW && vec) {
-        if (a.rows >= 512 && a.Kp <= 8 * 256) launch_k(quant_rows_vec_kernel<1>, dim3((unsigned)((a.rows + 3) / 4)), dim3(256), 0, st, a);
-        else launch_k(quant_rows_vec_kernel<4>, dim3((unsigned)a.rows), dim3(256), 0, st, a);
+        if (a.rows >= 512 && a.Kp <= 8 * 256)
+            launch_k(quant_rows_vec_kernel<1>, dim3((unsigned)((a.rows + 3) / 4) + more), dim3(256), 0, st, a);
+        else
+            launch_k(quant_rows_vec_kernel<4>, dim3((unsigned)a.rows + more), dim3(256), 0, st, a);
     } else if (a.mode == ACT_ROW) {
-        launch_k(quant_rows_kernel, dim3(a.rows), dim3(1024), 0, st, a);
+        launch_k(quant_rows_kernel, dim3((unsigned)a.rows + more), dim3(1024), 0, st, a);
     } else {
         const int nb = a.Kp / BLK;
-        launch_k(quant_blocks_kernel, dim3((unsigned)((nb + 63) / 64), (unsigned)a.rows), dim3(256), 0, st,
-                           a);
+        launch_k(quant_blocks_kernel, dim3((unsigned)((nb + 63) / 64), (unsigned)a.rows + more), dim3(256), 0, st, a);
     }
 }
 
@@ -307,67 +373,52 @@ void launch_combine_tok(float *out, const float *y, const int *tok_rows, const i
 // ---------------------------------------------------------------------------
 // The reference's own router (peregrine-model/src/router.rs:52-170, after
 // the router matmul), one wavefront per token: sigmoid scores (exp evaluated
-// as glibc expf), greedy top-k over score + bias with the same argmax rounds,
-// weight = the winner's sigmoid; unfilled slots (0, 0); the negligible tail
-// (router.rs:191-209) dropped when min_share > 0; optional renormalisation
-// over all k slots (+1e-20, summed in slot order); times routed_scale.
+// as glibc expf), greedy top-k over score + bias (route.h's selection over
+// packed keys), weight = the winner's sigmoid; unfilled slots (0, 0); the
+// negligible tail (router.rs:191-209) dropped when min_share > 0; optional
+// renormalisation over all k slots (+1e-20, summed in slot order); times
+// routed_scale. A chain of latencies at one token: sums read the slots as
+// scalars (readlane), the winners' sigmoids come from LDS (160 experts, top-8:
+// 7.0 -> 4.1 us against argmax rounds over values and indices).
 template <int PER>
 __global__ __launch_bounds__(64) void route_sigmoid_kernel(const float *logits, const float *bias, int E, int k,
                                                            int norm_topk, float routed_scale, float min_share,
                                                            int *ids_out, float *w_out, int *keff_out) {
+    __shared__ float sgl[PER * 64];
     const int s = blockIdx.x, lane = threadIdx.x & 63;
     const float *l = logits + (size_t)s * E;
-    float ve[PER], sg[PER];
+    const ExpTab tab = exp_tab();
+    float lv[PER], bv[PER];
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+        const int e = min(lane + 64 * j, E - 1);
+        lv[j] = l[e];
+        bv[j] = bias ? bias[e] : 0.0f;
+    }
+    uint64_t kv[PER];
 #pragma unroll
     for (int j = 0; j < PER; j++) {
         const int e = lane + 64 * j;
-        float c = -INFINITY, sig = 0.0f;
-        if (e < E) {
-            sig = __fdiv_rn(1.0f, __fadd_rn(1.0f, expf_glibc(-l[e])));
-            c = __fadd_rn(sig, bias ? bias[e] : 0.0f);
-        }
-        sg[j] = sig;
-        ve[j] = c > -INFINITY ? c : -INFINITY;   // NaN and -inf never qualify
+        const float sig = __fdiv_rn(1.0f, __fadd_rn(1.0f, expf_wave(-lv[j], tab)));
+        kv[j] = e < E ? route_key(__fadd_rn(sig, bv[j]), e) : 0;   // NaN and -inf never qualify
+        sgl[e] = sig;
     }
-    float myw = 0.0f;
-    int myid = 0, kept = 0;
-    for (int kk = 0; kk < k; kk++) {
-        float bv = -INFINITY;
-        int bi = 0x7fffffff;
-#pragma unroll
-        for (int j = 0; j < PER; j++)
-            if (ve[j] > bv) {
-                bv = ve[j];
-                bi = lane + 64 * j;
-            }
-        wave_argmax(bv, bi);
-        if (!(bv > -INFINITY)) break;   // uniform: nothing valid remains
-        float cand = 0.0f;
-#pragma unroll
-        for (int j = 0; j < PER; j++)
-            if (j == (bi >> 6)) cand = sg[j];
-        const float wsel = __shfl(cand, bi & 63);   // the winner's sigmoid
-        if (lane == kk) {
-            myw = wsel;
-            myid = bi;
-        }
-        if ((bi & 63) == lane) {
-#pragma unroll
-            for (int j = 0; j < PER; j++)
-                if (j == (bi >> 6)) ve[j] = -INFINITY;
-        }
-        kept++;
-    }
+    __syncthreads();
+    uint64_t mykey, top;
+    int kept;
+    route_select_keys<PER>(kv, k, mykey, kept, top);
+    int myid = lane < kept ? route_key_index(mykey) : 0;
+    float myw = lane < kept ? sgl[myid] : 0.0f;
+    auto slot = [&](int i) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(myw), i)); };
     // negligible tail: a trailing run of kept weights under min_share of the
     // kept sum, at most kept - 1 (every lane computes the same, uniformly)
     int drop = 0;
     if (min_share > 0.0f && kept > 1) {
         float sum = 0.0f;
-        for (int i = 0; i < kept; i++) sum = __fadd_rn(sum, __shfl(myw, i));
+        for (int i = 0; i < kept; i++) sum = __fadd_rn(sum, slot(i));
         if (isfinite(sum) && sum > 0.0f) {
             while (drop < kept - 1) {
-                const float wi = __shfl(myw, kept - 1 - drop);
-                if (__fdiv_rn(wi, sum) >= min_share) break;
+                if (__fdiv_rn(slot(kept - 1 - drop), sum) >= min_share) break;
                 drop++;
             }
         }
@@ -379,7 +430,7 @@ __global__ __launch_bounds__(64) void route_sigmoid_kernel(const float *logits, 
     }
     if (norm_topk) {
         float sm = 0.0f;
-        for (int i = 0; i < k; i++) sm = __fadd_rn(sm, __shfl(myw, i));
+        for (int i = 0; i < k; i++) sm = __fadd_rn(sm, slot(i));
         sm = __fadd_rn(sm, 1e-20f);
         myw = __fdiv_rn(myw, sm);
     }

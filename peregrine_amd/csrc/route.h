@@ -12,39 +12,6 @@ namespace phip {
 // then w_j = exp(l_j - l_0) / sum_j exp(l_j - l_0) summed in selection order.
 // One wavefront per token.
 // ---------------------------------------------------------------------------
-// (value desc, index asc) maximum across the wavefront, returned uniform.
-// DPP exchanges inside each row of 16 lanes (quad swaps, half-row and row
-// mirrors leave all 16 lanes agreeing), then the four row results are read
-// as scalars.
-template <int CTRL>
-__device__ __forceinline__ void argmax_dpp(float &v, int &i) {
-    const float ov = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
-    const int oi = __builtin_amdgcn_update_dpp(0, i, CTRL, 0xF, 0xF, false);
-    if (ov > v || (ov == v && oi < i)) {
-        v = ov;
-        i = oi;
-    }
-}
-__device__ __forceinline__ void wave_argmax(float &v, int &i) {
-    argmax_dpp<0xB1>(v, i);    // quad_perm [1,0,3,2]
-    argmax_dpp<0x4E>(v, i);    // quad_perm [2,3,0,1]
-    argmax_dpp<0x141>(v, i);   // row_half_mirror
-    argmax_dpp<0x140>(v, i);   // row_mirror
-    float bv = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 0));
-    int bi = __builtin_amdgcn_readlane(i, 0);
-#pragma unroll
-    for (int r = 16; r < 64; r += 16) {
-        const float rv = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), r));
-        const int ri = __builtin_amdgcn_readlane(i, r);
-        if (rv > bv || (rv == bv && ri < bi)) {
-            bv = rv;
-            bi = ri;
-        }
-    }
-    v = bv;
-    i = bi;
-}
-
 // (value desc, index asc) as one unsigned 64-bit key: the high word orders
 // floats as integers (sign-folded, -0 folded onto +0), the low word is the
 // complemented index, so a larger key is a larger value or, at equal values,
@@ -102,15 +69,9 @@ __device__ __forceinline__ void sort_keys_desc(uint64_t (&kv)[PER]) {
 // remaining slots empty. Lane kk returns the kk-th pick's key in mykey; kept
 // and first (the top key) are uniform.
 template <int PER>
-__device__ __forceinline__ void route_select(const float *l, int E, int k, uint64_t &mykey, int &kept,
-                                             uint64_t &first) {
+__device__ __forceinline__ void route_select_keys(uint64_t (&kv)[PER], int k, uint64_t &mykey, int &kept,
+                                                  uint64_t &first) {
     const int lane = threadIdx.x & 63;
-    uint64_t kv[PER];
-#pragma unroll
-    for (int j = 0; j < PER; j++) {
-        const int e = lane + 64 * j;
-        kv[j] = e < E ? route_key(l[e], e) : 0;
-    }
     sort_keys_desc<PER>(kv);
     mykey = 0;
     first = 0;
@@ -136,6 +97,19 @@ __device__ __forceinline__ void route_select(const float *l, int E, int k, uint6
         }
         kept++;
     }
+}
+
+template <int PER>
+__device__ __forceinline__ void route_select(const float *l, int E, int k, uint64_t &mykey, int &kept,
+                                             uint64_t &first) {
+    const int lane = threadIdx.x & 63;
+    uint64_t kv[PER];
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+        const int e = lane + 64 * j;
+        kv[j] = e < E ? route_key(l[e], e) : 0;
+    }
+    route_select_keys<PER>(kv, k, mykey, kept, first);
 }
 
 // Slot ids and softmax weights from a selection: empty slots get id 0 and

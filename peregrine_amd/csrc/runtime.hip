@@ -695,7 +695,11 @@ struct DispatchOpts {
     int lead_bound = 0;                 // > 0: the plan lists leading tiles, at most this many
     const float *combine_w = nullptr;   // one token: down + combine in one launch, weights [k]
     float *combine_out = nullptr;       //   and the layer output [D]
+    const int *one_ids = nullptr;       // one token's ids: the activation quantisation also builds its table
+    int one_k = 0, one_E = 0;
+    TableOut one_t{};
     const float *tail_w = nullptr;      // one token: the down GEMV's last workgroup per tile combines
+    const int *tail_kk = nullptr;
     float *tail_out = nullptr;
     int *tail_ctr = nullptr;    // host-buffer calls: the activation quantisation also stages this metadata
     const void *meta_src = nullptr;
@@ -746,7 +750,8 @@ void run_experts(Ctx *c, Prof &prof, const ExpertDesc *desc, const RowPlan &plan
     const int act = epi_act(ga);
     if (!opt.x_quantized) {
         QuantArgs qa{x_dev, gg.K, rows_x, gg.K, gg.Kp, s.xq, s.xs, s.sx, s.sxs, act,
-                     (const uint4 *)opt.meta_src, (uint4 *)opt.meta_dst, opt.meta_n16};
+                     (const uint4 *)opt.meta_src, (uint4 *)opt.meta_dst, opt.meta_n16,
+                     opt.one_ids, opt.one_k, opt.one_E, opt.one_t};
         prof.mark(COLI_HIP_K_QUANT_X);
         launch_quant_rows(qa, c->stream);
         if (opt.after_quant) hipEventRecord(opt.after_quant, c->stream);
@@ -781,7 +786,10 @@ void run_experts(Ctx *c, Prof &prof, const ExpertDesc *desc, const RowPlan &plan
     else
         launch_mfma_gateup(da, gg, act, T_bound, c->stream);
 
-    if (act == ACT_ROW) {
+    // per-row weights: the down GEMV's workgroups quantise their row of h
+    const bool h_in_down = act == ACT_ROW && arm == COLI_HIP_ARM_GEMV && !opt.combine_out && opt.split_dn.split <= 1 &&
+                           !g_dbg_dn && gemv_row_ok(gd);
+    if (act == ACT_ROW && !h_in_down) {
         // h's columns up to Kp are written too (zero weights: zeros), so the
         // rows are whole aligned groups whatever I is
         QuantArgs qh{s.h, s.hs, R_bound, gd.Kp, gd.Kp, s.hq, s.hqs, s.sh, s.shs, ACT_ROW};
@@ -804,6 +812,9 @@ void run_experts(Ctx *c, Prof &prof, const ExpertDesc *desc, const RowPlan &plan
     dd.route = RouteArgs{};
     dd.tail_out = opt.tail_out;
     dd.tail_w = opt.tail_w;
+    dd.tail_kk = opt.tail_kk;
+    dd.hf = h_in_down ? s.h : nullptr;
+    dd.hf_stride = s.hs;
     dd.tail_ctr = opt.tail_ctr;
     apply_split(dd, arm == COLI_HIP_ARM_GEMV ? opt.split_dn : GemvSplit{}, opt);
     prof.mark(COLI_HIP_K_DOWN);
@@ -1707,7 +1718,8 @@ int moe_forward_impl(const ColiHipExpertSet *set, const float *x_dev, int S, con
         opt.combine_out = out_dev;
     }
     // otherwise, one token: the down GEMV's tail does the combine
-    const bool tail_c = one_token && !fuse_dc && tail_combine_on() && !g_dbg_dn && k <= GEMV_TAIL_MAXK &&
+    const bool one_ids = S == 1 && arm == COLI_HIP_ARM_GEMV && !logits_dev;   // its table: built with the quantisation
+    const bool tail_c = (one_token || one_ids) && !fuse_dc && tail_combine_on() && !g_dbg_dn && k <= GEMV_TAIL_MAXK &&
                         (gd.O + 63) / 64 <= GEMV_TAIL_TILES;
     if (tail_c) {
         opt.tail_w = w_dev;
@@ -1725,7 +1737,14 @@ int moe_forward_impl(const ColiHipExpertSet *set, const float *x_dev, int S, con
         opt.n_rows_fixed = k;
     } else {
         prof.mark(COLI_HIP_K_TABLE);
-        launch_build_table(ids_dev, S, k, E, t, tmax, tbl_work, c->stream);
+        if (one_ids) {
+            opt.one_ids = ids_dev;
+            opt.one_k = k;
+            opt.one_E = E;
+            opt.one_t = t;
+            opt.act_zero = true;
+            opt.tail_kk = t.row_kk;
+        } else launch_build_table(ids_dev, S, k, E, t, tmax, tbl_work, c->stream);
         plan.row_exp = t.row_exp;
         plan.row_act = t.row_tok;
         plan.mt_exp = t.mt_exp;
