@@ -599,8 +599,12 @@ struct SaStage {
     static constexpr int BYTES = S + 8 * 128;
 };
 
+// Grouped weights with per-row activations (EPI_GRP) are held to 168 VGPRs, so
+// three workgroups share a CU (172 otherwise: two). 160 experts, D = 5120,
+// I = 1536, gs = 128: 64 tokens 365 -> 329 us, 700 tokens 843 -> 762 us; gs = 32,
+// 64 tokens 426 -> 382 us.
 template <bool W4, int EPI, bool GATEUP, int PD, bool WNT, bool XO = false>
-__global__ __launch_bounds__(256) void mfma_sa_kernel(DotArgs a, MatGeom g) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EPI == EPI_GRP ? 3 : 1))) void mfma_sa_kernel(DotArgs a, MatGeom g) {
     constexpr int NSUB = 2;
     typedef SaStage<W4> ST;
     constexpr int NSTG = PD + 2;   // stage b-2 is refilled once every wave is past block b-1's barrier
