@@ -839,6 +839,25 @@ bool row_groups(const MatGeom &gg, const MatGeom &gd, int R, int n, int ga) {
     return (long)R >= 64L * n || ((long)R >= 24L * n && gg.nb >= 64);
 }
 
+// The arm of a dispatch of R rows when none is forced. The GEMV
+// reads an expert's weights once per row (again from the caches where rows
+// share it), the grouped GEMM once per expert, but a workgroup of the GEMM
+// walks all of K block by block: 75 us at D = 5120 however little there is to
+// read. Measured, layer times GEMV / GEMM in us. 160 experts, D = 5120, I =
+// 1536, top-8: int4 gs = 32 16 rows 56 / 79, 40 rows 107 / 114 (skewed
+// popularity 94 / 99), 48 rows 120 / 141 (skewed 102 / 98); per row 32 rows 79 /
+// 88; gs = 128 48 rows 115 / 147; int8 16 rows 94 / 98, 24 rows 135 / 133 (skewed
+// 128 / 102). 256 experts, D = 6144, I = 2048: int4 40 rows 162 / 181 (skewed 144
+// / 137), int8 16 rows 128 / 121. Small layers: 16 experts, D = 2048, I = 768, 32
+// rows int4 33 / 44, 24 rows int8 45 / 45; 64 experts, D = 1024, I = 512, 48 rows
+// int4 30 / 35, 36 rows int8 36 / 35. Sharing does not turn it round: 1 expert,
+// D = 5120, 16 rows int4 37 / 90, int8 59 / 68; 4 experts, D = 2048, 32 rows 28 / 47.
+bool gemv_pays(const MatGeom &gg, const MatGeom &gd, int R) {
+    const double bytes = (double)gg.Op * gg.Kp * (gg.w4 ? 1.0 : 2.0) + (double)gd.Op * gd.Kp * (gd.w4 ? 0.5 : 1.0);   // one expert's weights
+    if (gg.w4 && gd.w4) return R <= (bytes <= 4e6 ? 48 : bytes <= 12e6 ? 40 : 32);
+    return R <= (bytes <= 4e6 ? 24 : bytes <= 25e6 ? 16 : 8);
+}
+
 struct ReduceSpec {
     const int *row_ptr, *row_idx;
     const float *rw;
@@ -996,7 +1015,8 @@ int expert_group_impl(ColiHipTensor *const *gates, ColiHipTensor *const *ups, Co
     if (!select_ctx(c)) return 0;
     const int D = gg.K, ga = act_group();
     int arm = forced_arm();
-    if (arm < 0) arm = max_rows <= 1 ? COLI_HIP_ARM_GEMV : COLI_HIP_ARM_MFMA;
+    // (calls that report their arm keep the simple rule)
+    if (arm < 0) arm = max_rows <= 1 || (!arm_out && gemv_pays(gg, gd, total)) ? COLI_HIP_ARM_GEMV : COLI_HIP_ARM_MFMA;
     if (arm_out) *arm_out = arm;
 
     // host-built plan: descriptors in call order, rows consecutive
@@ -1609,8 +1629,8 @@ int moe_forward_impl(const ColiHipExpertSet *set, const float *x_dev, int S, con
     const int tmax = (R + MT_ROWS - 1) / MT_ROWS + std::min(E, R);
     const int lead_max = mmap::row_lead_bound(R, std::min(E, R));
     if (arm < 0) arm = forced_arm();
-    if (arm < 0) arm = S == 1 ? COLI_HIP_ARM_GEMV : COLI_HIP_ARM_MFMA;
     const MatGeom &gg = set->gg, &gd = set->gd;
+    if (arm < 0) arm = S == 1 || gemv_pays(gg, gd, R) ? COLI_HIP_ARM_GEMV : COLI_HIP_ARM_MFMA;
 
     // table layout in one buffer
     const size_t n_int =
