@@ -1175,22 +1175,11 @@ static void launch_mfma_dma(const DotArgs &a, const MatGeom &g, int grid_tiles, 
     if constexpr (W4) {
         // weight-reuse dispatches in the XCD-aware expert-major order: config 4
         // gate/up fetch 3.69 -> 2.60 GB, down 1.50 -> 1.01 GB, step 1.5% faster
-        // (per-row weights with as many rows run mfma_row_kernel)
-        if constexpr (EPI != EPI_ROW) {
-            if (a.w_reuse) {
-                launch_mfma_sa_h<W4, EPI, GATEUP, PD, false, true>(a, g, grid_tiles, st);
-                return;
-            }
-        }
-        launch_mfma_sa_h<W4, EPI, GATEUP, PD, true>(a, g, grid_tiles, st);
+        if (a.w_reuse) launch_mfma_sa_h<W4, EPI, GATEUP, PD, false, true>(a, g, grid_tiles, st);
+        else launch_mfma_sa_h<W4, EPI, GATEUP, PD, true>(a, g, grid_tiles, st);
     } else {
-        if constexpr (EPI != EPI_ROW) {
-            if (a.w_reuse) {
-                launch_mfma_dma_h<W4, EPI, GATEUP, PD, false>(a, g, grid_tiles, st);
-                return;
-            }
-        }
-        launch_mfma_dma_h<W4, EPI, GATEUP, PD, true>(a, g, grid_tiles, st);
+        if (a.w_reuse) launch_mfma_dma_h<W4, EPI, GATEUP, PD, false>(a, g, grid_tiles, st);
+        else launch_mfma_dma_h<W4, EPI, GATEUP, PD, true>(a, g, grid_tiles, st);
     }
 }
 

@@ -833,10 +833,16 @@ void run_experts(Ctx *c, Prof &prof, const ExpertDesc *desc, const RowPlan &plan
 // the 32-row kernel -> this one: 12.8 rows per expert (uniform routing) 387 ->
 // 414 us, 25.6 rows 475 -> 455, 51 rows 859 -> 538; skewed routing 25.6 rows
 // 563 -> 485, 89 rows 944 -> 745. With a short K its start and end weigh more
-// (K = 1000, 30 rows per expert: 71 -> 74 us), so there from 64 rows on.
+// (K = 1000, 30 rows per expert, int4 71 -> 74 us), so there from 64 rows on,
+// or for int8 with many items (128 experts, K = 1536, 31 rows 134 -> 119 us).
+// And it needs items to fill the chip: 13 x 12 of them, int4 (8 experts, D =
+// 4096, 150 rows each) 101 -> 110 us, int8 128 -> 118; 20 x 2 53 -> 57 us; 35 x 6
+// 92 -> 89.
 bool row_groups(const MatGeom &gg, const MatGeom &gd, int R, int n, int ga) {
     if (epi_act(ga) != ACT_ROW || !(gg.per_row || gd.per_row)) return false;
-    return (long)R >= 64L * n || ((long)R >= 24L * n && gg.nb >= 64);
+    const long items = (long)mmap::row_lead_bound(R, n) * mmap::slab_count(true, gg.O);
+    const bool many = (long)R >= (gg.nb >= 64 ? 24L : 64L) * n && items >= (gg.w4 ? 256 : 128);
+    return many || (!gg.w4 && (long)R >= 24L * n && items >= 512);
 }
 
 // The arm of a dispatch of R rows when none is forced. The GEMV

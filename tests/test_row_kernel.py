@@ -82,9 +82,14 @@ def test_row_checker_is_not_vacuous(chk):
     assert run_check(chk, True, True, 96, 64, [40] * 9, lead_bound=8) > 0   # the last tile's item is missing
 
 
+def reaches_row_kernel(R, n, D, I):
+    """The dispatch rule (int4's, the narrower): rows per expert and items."""
+    return R >= (24 if D > 2016 else 64) * n and (R // 128 + n) * -(-(-(-I // 32) * 32) // 128) >= 256
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("fmt", [qt.FMT_I4, qt.FMT_I8])
-@pytest.mark.parametrize("D,I", [(1536, 640), (1000, 713), (160, 33), (96, 64)])
+@pytest.mark.parametrize("D,I", [(1000, 8130), (160, 8161), (96, 8192)])
 @pytest.mark.parametrize("rows", [[200, 1, 31, 95], [129, 128], [64, 97, 288]])
 def test_row_kernel_matches_oracle(hip, orc, fmt, D, I, rows):
     print("row kernel", fmt, D, I, rows, flush=True)
@@ -94,7 +99,7 @@ def test_row_kernel_matches_oracle(hip, orc, fmt, D, I, rows):
         trip = synth.make_expert(rng, D, I, fmt, 32)
         gpu.append(hip.GpuExpert.upload_grouped(0, trip[0][:2], trip[1][:2], trip[2][:2], D, I, fmt, 32))
         ora.append(tuple(orc.Tensor(t[0], t[1], fmt, i, o, 32) for t, (o, i) in zip(trip, ((I, D), (I, D), (D, I)))))
-    assert sum(rows) >= 64 * len(rows)   # the dispatch rule of the kernel at any K
+    assert reaches_row_kernel(sum(rows), len(rows), D, I)
     x = rng.standard_normal((sum(rows), D)).astype(np.float32)
     hip.set_act_group(0)
     hip.set_arm(0)
@@ -111,13 +116,13 @@ def test_row_kernel_matches_oracle(hip, orc, fmt, D, I, rows):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("fmt", [qt.FMT_I4, qt.FMT_I8])
-@pytest.mark.parametrize("E,S,k", [(5, 64, 3), (9, 300, 4), (3, 700, 3)])
-def test_row_kernel_layer(hip, orc, fmt, E, S, k):
+@pytest.mark.parametrize("E,S,k,D,I", [(5, 64, 3, 2048, 5440), (9, 300, 4, 2048, 1900), (3, 700, 3, 96, 1800)])
+def test_row_kernel_layer(hip, orc, fmt, E, S, k, D, I):
     """The layer, whose leading tiles the device table lists (both table
     forms), with ids that skip an expert, repeat one and leave the range; at
     D = 2048 the rule's lower bound of 24 rows per expert holds too."""
     print("row layer", fmt, E, S, k, flush=True)
-    D, I = 2048, 96
+    assert reaches_row_kernel(S * k, E, D, I)
     rng = np.random.default_rng(E * S + fmt)
     gpu, ora = [], []
     for _ in range(E):
