@@ -1083,7 +1083,6 @@ int expert_group_impl(ColiHipTensor *const *gates, ColiHipTensor *const *ups, Co
         std::memcpy(ri, red->row_idx, (size_t)total * 4);
         std::memcpy(rwv, red->rw, (size_t)total * 4);
     }
-    std::memcpy(c->pin_x.p, x, xb);
 
     uint8_t *dm = (uint8_t *)c->meta.p;
     int *di = (int *)(dm + desc_b);
@@ -1145,7 +1144,14 @@ int expert_group_impl(ColiHipTensor *const *gates, ColiHipTensor *const *ups, Co
     };
 
     const bool graphs_on = graph_cache_enabled();
-    if (graphs_on && !profile && !g_dbg_gu && !g_dbg_dn) {
+    // Large x, run eagerly: staged in chunks of rows, each quantised (read
+    // across PCIe) while the host copies the next. 96 rows of 5120 (2 MB): call
+    // 243 -> 216 us; 192 rows 427 -> 393 (two chunks 406, three 391); 480 rows 868
+    // -> 722 (two chunks 780, three 743).
+    const bool cached = graphs_on && !profile && !g_dbg_gu && !g_dbg_dn;
+    const int n_chunk = cached || profile ? 1 : (int)std::min<size_t>(8, xb >> 19);
+    if (n_chunk <= 1) std::memcpy(c->pin_x.p, x, xb);
+    if (cached) {
         const ColiHipTensor *g0 = gates[0], *d0 = downs[0];
         ShapeKey key;
         shape_key(&key, {arm, count, D, gg.O, s_n, ga, g0->fmt, g0->gs, d0->fmt, d0->gs, g_spin_limit, gemv_split_target()},
@@ -1216,6 +1222,15 @@ int expert_group_impl(ColiHipTensor *const *gates, ColiHipTensor *const *ups, Co
     bool phases = profile;
     for (auto &e : c->phase_ev)
         if (phases && !e && hipEventCreateWithFlags(&e, hipEventDisableSystemFence) != hipSuccess) phases = false;
+    for (int i = 0; n_chunk > 1 && i < n_chunk; i++) {
+        const int r0 = (int)((long)total * i / n_chunk), r1 = (int)((long)total * (i + 1) / n_chunk);
+        std::memcpy((float *)c->pin_x.p + (size_t)r0 * D, x + (size_t)r0 * D, (size_t)(r1 - r0) * D * 4);
+        launch_quant_rows(QuantArgs{x_dev + (size_t)r0 * D, D, r1 - r0, D, gg.Kp, s.xq + (size_t)r0 * s.xs, s.xs,
+                                    s.sx + (size_t)r0 * s.sxs, s.sxs, epi_act(ga), (const uint4 *)opt.meta_src,
+                                    (uint4 *)opt.meta_dst, opt.meta_n16},
+                          c->stream);
+        opt.x_quantized = true;
+    }
     if (!enqueue(prof, phases) || !hip_ok(hipStreamSynchronize(c->stream), "expert group synchronize")) return 0;
     prof.finish();
     if (phases) {
