@@ -1648,14 +1648,14 @@ int moe_forward_impl(const ColiHipExpertSet *set, const float *x_dev, int S, con
     if (!select_ctx(c)) return 0;
     const int E = set->count, R = S * k;
     const int tmax = (R + MT_ROWS - 1) / MT_ROWS + std::min(E, R);
-    const int lead_max = mmap::row_lead_bound(R, std::min(E, R));
     if (arm < 0) arm = forced_arm();
     const MatGeom &gg = set->gg, &gd = set->gd;
     if (arm < 0) arm = S == 1 || gemv_pays(gg, gd, R) ? COLI_HIP_ARM_GEMV : COLI_HIP_ARM_MFMA;
 
-    // table layout in one buffer
-    const size_t n_int =
-        4 + (size_t)E + (E + 1) + 3 * (size_t)R + 2 * (size_t)R + 4 * (size_t)tmax + (size_t)lead_max + table_work_ints(S, k, E);
+    // table layout in one buffer (the leading tiles last: the no-allocation
+    // call does without them rather than be refused for them)
+    int lead_max = arm == COLI_HIP_ARM_MFMA && row_groups(gg, gd, R, E, ga) ? mmap::row_lead_bound(R, std::min(E, R)) : 0;
+    const size_t n_int = 4 + (size_t)E + (E + 1) + 3 * (size_t)R + 2 * (size_t)R + 4 * (size_t)tmax + table_work_ints(S, k, E);
     Scratch s{};
     int *p = nullptr;
     if (fixed_scratch) {
@@ -1665,7 +1665,8 @@ int moe_forward_impl(const ColiHipExpertSet *set, const float *x_dev, int S, con
         size_t need = 0;
         if (!carve_rows(gg, gd, S, R, ga, nullptr, &need, &s)) return 0;
         const size_t tbl_off = need;
-        need += round_up(n_int * 4, 256);
+        if (tbl_off + round_up((n_int + lead_max) * 4, 256) > COLI_HIP_FIXED_SCRATCH_BYTES) lead_max = 0;
+        need += round_up((n_int + lead_max) * 4, 256);
         if (need > COLI_HIP_FIXED_SCRATCH_BYTES) {
             std::fprintf(stderr,
                          "[HIP] moe_forward (no allocation): this call needs %zu bytes of scratch, more than the "
@@ -1676,7 +1677,7 @@ int moe_forward_impl(const ColiHipExpertSet *set, const float *x_dev, int S, con
         carve_rows(gg, gd, S, R, ga, c->fixed_scratch, &need, &s);
         p = (int *)(c->fixed_scratch + tbl_off);
     } else {
-        if (!reserve_rows(c, gg, gd, S, R, ga, &s) || !reserve(c, c->tbl, n_int * 4)) return 0;
+        if (!reserve_rows(c, gg, gd, S, R, ga, &s) || !reserve(c, c->tbl, (n_int + lead_max) * 4)) return 0;
         p = (int *)c->tbl.p;
     }
     TableOut t{};
@@ -1704,9 +1705,8 @@ int moe_forward_impl(const ColiHipExpertSet *set, const float *x_dev, int S, con
     p += tmax;
     t.mt_first = p;
     p += tmax;
-    int *lead = p;
-    p += lead_max;
     int *tbl_work = p;
+    int *lead = p + table_work_ints(S, k, E);
     c->tbl_view = t;
     c->tbl_E = E;
     c->tbl_R = R;
@@ -1715,7 +1715,7 @@ int moe_forward_impl(const ColiHipExpertSet *set, const float *x_dev, int S, con
     if (fixed_scratch) prof.on = false;   // profiling creates events: not on the no-allocation path
     DispatchOpts opt;
     opt.w_reuse = R >= 2 * MT_ROWS * E;   // about two or more M tiles per expert
-    if (row_groups(gg, gd, R, E, ga)) {
+    if (lead_max > 0) {
         t.lead = lead;
         opt.lead_bound = lead_max;
     }
