@@ -311,6 +311,7 @@ struct DotArgs {   // shared by the GEMV and MFMA arms
     int spin_limit;                                                     // GEMV: polls before a bounded wait gives up
     int *wait_failed;                                                   // GEMV: host-visible word, set to 1 when one does
     int w_reuse;                                                        // MFMA arm: M tiles re-read each expert's weights
+    int x_rows;                                                         // MFMA arm: rows of xq (its launch checks their bytes)
     int lead_bound;                                                     // > 0: per-row weights run mfma_row_kernel, G <= this
     RouteArgs route;                                                    // gate/up GEMV: logits != null -> fused router
     // down GEMV, one token (rows 0..n-1 in top-k order): the last workgroup

@@ -644,7 +644,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EPI == EPI_
     // ---- copy sources: uniform bases + per-lane offsets ----
     // A: a dword of row 8*wave + lane/8 (rows past the expert's end repeat
     // its last row; never stored)
-    const uint32_t voff_a = (uint32_t)act_row(mmap::a_row(r0, rend, wave, lane)) * (uint32_t)a.x_stride + mmap::a_col(lane);
+    const uint32_t voff_a = mmap::x_off32(act_row(mmap::a_row(r0, rend, wave, lane)), a.x_stride) + mmap::a_col(lane);
     const uint8_t *base_a = uniform_ptr(a.xq);
     // weights and their scales: this wave's two subtiles 2w, 2w+1 (one
     // tensor), lane half hh -> subtile 2w + hh; tiles past the tensor clamp
@@ -931,7 +931,7 @@ __device__ __forceinline__ void mfma_row_body(const DotArgs &a, const MatGeom &g
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         const int r = mmap::row_of(has_a ? wave : 0, i, lane), rr = min(r0 + r, rend - 1);
-        const uint32_t at = (uint32_t)act_row(rr) * (uint32_t)a.x_stride;
+        const uint32_t at = mmap::x_off32(act_row(rr), a.x_stride);
         const int p = mmap::row_piece(r, lane & 3);
         voff_a[i] = at + mmap::row_col(p, false);
         voff_a1[i] = at + mmap::row_col(p, true);
@@ -1194,23 +1194,29 @@ static int mfma_mode() {
 template <bool W4, int EPI, bool GATEUP>
 static void launch_mfma_t(const DotArgs &a, const MatGeom &g, int grid_tiles, hipStream_t st) {
     const int m = mfma_mode();
-    if (!a.dots && m != 0) {
+    // 32-bit copy offsets: the staged kernels need one matrix's weights within
+    // 4 GiB, the scalar-base ones (int4's, mfma_row_kernel) the activation
+    // codes too; beyond that, the next kernel with 64-bit addresses
+    const bool w32 = mmap::off32_ok((uint64_t)g.Op * g.nb * (W4 ? 16 : 32));
+    const bool x32 = mmap::off32_ok((uint64_t)a.x_rows * a.x_stride);
+    if (!a.dots && m != 0 && w32) {
         if constexpr (EPI == EPI_ROW) {
-            if (a.lead_bound > 0) {
+            if (a.lead_bound > 0 && x32) {
                 launch_mfma_row<W4, GATEUP>(a, g, st);
                 return;
             }
         }
-        if (mfma_dma_lds<W4, EPI, DMA_PD_SHALLOW>(g) <= 160 * 1024 / 3) {
+        const bool staged = !W4 || x32;
+        if (staged && mfma_dma_lds<W4, EPI, DMA_PD_SHALLOW>(g) <= 160 * 1024 / 3) {
             launch_mfma_dma<W4, EPI, GATEUP, DMA_PD_SHALLOW>(a, g, grid_tiles, st);
             return;
         }
-        if (mfma_dma_lds<W4, EPI, DMA_PD_NARROW>(g) <= 160 * 1024 / 3) {
+        if (staged && mfma_dma_lds<W4, EPI, DMA_PD_NARROW>(g) <= 160 * 1024 / 3) {
             launch_mfma_dma<W4, EPI, GATEUP, DMA_PD_NARROW>(a, g, grid_tiles, st);
             return;
         }
         constexpr int PD = W4 ? DMA_PD_DEEP_W4 : DMA_PD_W8;
-        if (mfma_dma_lds<W4, EPI, PD>(g) <= 80 * 1024) {
+        if (staged && mfma_dma_lds<W4, EPI, PD>(g) <= 80 * 1024) {
             launch_mfma_dma<W4, EPI, GATEUP, PD>(a, g, grid_tiles, st);
             return;
         }

@@ -60,6 +60,12 @@ MMAP_HD void xo_place(int item, int NS, int ts, int nt, int *slab, int *tile) {
 
 // ---- copy sources ----------------------------------------------------------
 
+// Scalar-base copies (mfma_sa_kernel, mfma_row_kernel) address activation rows
+// and weight tiles by 32-bit offsets from one base: a buffer of more than 4
+// GiB is not theirs (off32_ok, checked where they are launched).
+MMAP_HD bool off32_ok(uint64_t bytes) { return bytes <= ((uint64_t)1 << 32); }
+MMAP_HD uint32_t x_off32(int row, int x_stride) { return (uint32_t)row * (uint32_t)x_stride; }
+
 // The activation dword a lane copies each block: row 8*wave + lane/8 of the
 // tile (rows past the expert's end repeat its last row, never stored),
 // column byte 4*(lane%8) of the 32-byte block.

@@ -761,6 +761,7 @@ void run_experts(Ctx *c, Prof &prof, const ExpertDesc *desc, const RowPlan &plan
     da.desc = desc;
     da.plan = plan;
     da.xq = s.xq;
+    da.x_rows = rows_x;
     da.x_stride = s.xs;
     da.sx = s.sx;
     da.sx_stride = s.sxs;
@@ -799,6 +800,7 @@ void run_experts(Ctx *c, Prof &prof, const ExpertDesc *desc, const RowPlan &plan
 
     DotArgs dd = da;
     dd.xq = s.hq;
+    dd.x_rows = R_bound;
     dd.x_stride = s.hqs;
     dd.sx = s.sh;
     dd.sx_stride = s.shs;

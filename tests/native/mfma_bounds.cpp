@@ -74,7 +74,10 @@ extern "C" long check_dispatch(int kind, int gateup, int xo, int b32, int grp_co
                     const int ra = a_row(r0, rend, wave, lane);
                     const int xr = act(ra);
                     need(xr >= 0 && xr < rows_x, "activation row", tile, ra, xr, rows_x);
-                    const long a0 = (long)xr * x_stride + a_col(lane);
+                    // mfma_sa_kernel's offset has 32 bits, mfma_dma_kernel's 64
+                    const long a0 = kind == 0 ? (long)(uint32_t)(x_off32(xr, x_stride) + a_col(lane))
+                                              : (long)xr * x_stride + a_col(lane);
+                    need(a0 == (long)xr * x_stride + a_col(lane), "activation offset wraps", tile, wave, lane, xr);
                     long w0[2] = {0, 0}, s0;
                     int nw = 1;
                     if (kind == 0) {
@@ -128,4 +131,5 @@ extern "C" long check_dispatch(int kind, int gateup, int xo, int b32, int grp_co
     return g_bad;
 }
 
+extern "C" int off32_ok_c(uint64_t bytes) { return off32_ok(bytes); }
 extern "C" int xo_item_c(int L, int n) { return xo_item(L, n); }

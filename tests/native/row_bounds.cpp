@@ -15,6 +15,7 @@ static void need(bool ok, const char *what, long a, long b, long c, long d) {
     if (!ok && g_bad++ < 8) std::fprintf(stderr, "row_bounds: %s (%ld %ld %ld %ld)\n", what, a, b, c, d);
 }
 
+extern "C" int off32_ok_c(uint64_t bytes) { return off32_ok(bytes); }
 extern "C" int row_lead_bound_c(int R, int n) { return row_lead_bound(R, n); }
 
 extern "C" long check_row_dispatch(int gateup, int w4, int nb, int O, int T, int lead_bound, const int *mt_exp,
@@ -53,8 +54,11 @@ extern "C" long check_row_dispatch(int gateup, int w4, int nb, int O, int T, int
                         need(p >= 0 && p < 2 * ROW_CB, "piece", r, lane, p, 0);
                         for (int c = 0; c < nc; ++c) {
                             const bool one = c * ROW_CB + 1 >= nb;
-                            const long col = (long)c * ROW_CB * BLK + row_col(p, one), at = (long)xr * x_stride + col;
-                            need(col + 16 <= (long)nb * BLK && at >= 0 && at + 16 <= x_bytes, "activation copy", tile, wave, lane, c);
+                            const long col = (long)c * ROW_CB * BLK + row_col(p, one);
+                            const uint32_t voff = x_off32(xr, x_stride) + row_col(p, one);   // as the kernel: 32 bits
+                            const long at = (long)c * ROW_CB * BLK + (long)voff;
+                            need(col + 16 <= (long)nb * BLK && at == (long)xr * x_stride + col && at + 16 <= x_bytes,
+                                 "activation copy", tile, wave, lane, c);
                         }
                     }
                     for (int t = 0; t < (w4 ? 1 : 2); ++t) {

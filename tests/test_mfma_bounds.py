@@ -149,6 +149,20 @@ def test_xo_order_is_a_bijection_for_every_item_count(chk):
         assert chk.xo_item_c(n, n) == -1
 
 
+@pytest.mark.parametrize("rows_x,K", [(524288, 8192), (524289, 8192), (838860, 5120), (838862, 5120)])
+def test_activation_offsets_reach_4gib(chk, rows_x, K):
+    """mfma_sa_kernel's 32-bit activation offsets hold exactly where its
+    launch accepts them; mfma_dma_kernel's have 64 bits."""
+    chk.off32_ok_c.argtypes = [ctypes.c_uint64]
+    tiles, R = tiles_from_groups([(0, 70)])
+    act = np.arange(rows_x - R, rows_x, dtype=np.int32)   # the last rows
+    T = len(tiles[0])
+    fits = bool(chk.off32_ok_c(rows_x * K))
+    assert fits == (rows_x * K <= 1 << 32)
+    assert (run_check(chk, 0, True, 0, 0, geom(K, 64, True, 0), tiles, R, T, act, rows_x, 1, True) == 0) == fits
+    assert run_check(chk, 1, True, 0, 0, geom(K, 64, False, 0), tiles, R, T, act, rows_x, 1, True) == 0
+
+
 def test_checker_is_not_vacuous(chk):
     """A dispatch that would read past a buffer or skip an item is reported:
     an activation buffer one row short, a tile whose rows run past R, and a

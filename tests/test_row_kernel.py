@@ -82,6 +82,21 @@ def test_row_checker_is_not_vacuous(chk):
     assert run_check(chk, True, True, 96, 64, [40] * 9, lead_bound=8) > 0   # the last tile's item is missing
 
 
+# the most rows within 4 GiB of activation codes, then the first whose offset needs a 33rd bit
+EDGE_4GIB = [(524288, 8192), (524289, 8192), (838860, 5120), (838862, 5120), (2796202, 1536), (2796204, 1536)]
+
+
+@pytest.mark.parametrize("rows_x,K", EDGE_4GIB)
+def test_row_kernel_offsets_reach_4gib(chk, rows_x, K):
+    """The kernel's 32-bit activation offsets hold exactly where its launch
+    accepts them."""
+    chk.off32_ok_c.argtypes = [ctypes.c_uint64]
+    act = np.arange(rows_x - 70, rows_x, dtype=np.int32)   # the last rows
+    for w4 in (True, False):
+        bad = run_check(chk, True, w4, K, 64, [70], row_act=act, rows_x=rows_x)
+        assert (bad == 0) == bool(chk.off32_ok_c(rows_x * K)) == (rows_x * K <= 1 << 32)
+
+
 def reaches_row_kernel(R, n, D, I):
     """The dispatch rule (int4's, the narrower): rows per expert and items."""
     return R >= (24 if D > 2016 else 64) * n and (R // 128 + n) * -(-(-(-I // 32) * 32) // 128) >= 256
