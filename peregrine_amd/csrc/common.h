@@ -97,8 +97,8 @@ struct RowPlan {
     const int *mt_row0;    // [T] first row of the tile
     const int *mt_rend;    // [T] one past the last row of that expert
     const int *mt_first;   // [T] the first M tile of that expert (its tiles are consecutive)
-    const int *lead;       // [G] leading M tiles of each expert's groups of four (mfma_row_kernel)
-    const int *counts;     // [4] {R, T, -, G} as built on the device (or host)
+    const int *lead;       // [1 + G] G, then the leading M tiles of each expert's groups of four (mfma_row_kernel)
+    const int *counts;     // [2] {R, T} as built on the device (or host)
     const ExpertDesc *row_desc;  // optional [R]: row r's descriptor, written by the router
 };
 
@@ -265,12 +265,12 @@ inline void launch_k(K kern, dim3 grid, dim3 block, size_t lds, hipStream_t st, 
 }
 
 struct TableOut {
-    int *hdr;          // [4]: R, T, n_u, G (0 without lead)
+    int *hdr;          // [4]: R, T, n_u, 0
     int *uexp, *off;   // [E], [E+1]
     int *row_tok, *row_kk, *row_exp;  // [R]
     int *tok_rows, *tok_kk;           // [S*k]: each token's rows in union order (-1 pads), their top-k slot
     int *mt_exp, *mt_row0, *mt_rend, *mt_first;  // [Tmax]
-    int *lead;                        // optional [row_lead_bound]: the leading M tiles (RowPlan.lead)
+    int *lead;                        // optional [1 + row_lead_bound]: the leading M tiles (RowPlan.lead)
 };
 
 struct QuantArgs {

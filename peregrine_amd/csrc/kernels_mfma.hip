@@ -1105,8 +1105,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void m
     if constexpr (GATEUP) tab = exp_tab();
     int slab, i;
     mmap::row_place((int)(blockIdx.x + gridDim.x * blockIdx.y), (int)gridDim.x, &slab, &i);
-    if (i >= a.plan.counts[3]) return;
-    const int tile = a.plan.lead[i];
+    if (i >= a.plan.lead[0]) return;
+    const int tile = a.plan.lead[1 + i];
     const int e = a.plan.mt_exp[tile], r0 = a.plan.mt_row0[tile];
     const int rend = min(a.plan.mt_rend[tile], r0 + mmap::ROW_TILES * MT_ROWS);
     const int nm = (rend - r0 + MT_ROWS - 1) / MT_ROWS;   // uniform

@@ -655,7 +655,8 @@ __device__ void table_offsets(int n_u, const int *uex, const int *cnt, int *base
                 t.hdr[0] = off + c;
                 t.hdr[1] = mt + (c + MT_ROWS - 1) / MT_ROWS;
                 t.hdr[2] = n_u;
-                t.hdr[3] = t.lead ? ld + nl : 0;
+                t.hdr[3] = 0;
+                if (t.lead) t.lead[0] = ld + nl;
             }
         }
         __syncthreads();
@@ -670,6 +671,7 @@ __device__ void table_offsets(int n_u, const int *uex, const int *cnt, int *base
         if (tid == 0) {
             t.off[0] = 0;
             t.hdr[0] = t.hdr[1] = t.hdr[2] = t.hdr[3] = 0;
+            if (t.lead) t.lead[0] = 0;
         }
         __syncthreads();
         return;
@@ -688,7 +690,7 @@ __device__ void table_offsets(int n_u, const int *uex, const int *cnt, int *base
         t.mt_row0[q] = offs[lo] + MT_ROWS * (q - mts[lo]);
         t.mt_rend[q] = offs[lo + 1];
         t.mt_first[q] = mts[lo];
-        if (t.lead && mmap::row_leads(q, mts[lo])) t.lead[lds[lo] + (q - mts[lo]) / LT] = q;
+        if (t.lead && mmap::row_leads(q, mts[lo])) t.lead[1 + lds[lo] + (q - mts[lo]) / LT] = q;
     }
     __syncthreads();
 }

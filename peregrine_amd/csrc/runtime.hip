@@ -1031,7 +1031,7 @@ int expert_group_impl(ColiHipTensor *const *gates, ColiHipTensor *const *ups, Co
     int T = 0;
     for (int i = 0; i < count; i++) T += (rows[i] + MT_ROWS - 1) / MT_ROWS;
     const int s_n = red ? red->s_n : 0;
-    const size_t n_int = (size_t)total /*row_exp*/ + 5 * (size_t)T + 4 + (red ? (size_t)(s_n + 1) + total : 0);
+    const size_t n_int = (size_t)total /*row_exp*/ + 5 * (size_t)T + 3 + (red ? (size_t)(s_n + 1) + total : 0);
     const size_t desc_b = round_up((size_t)count * sizeof(ExpertDesc), 16);
     // (a whole number of 16-byte words: the quantisation kernel stages it)
     const size_t meta_b = round_up(desc_b + n_int * 4 + (red ? (size_t)total * 4 : 0), 16);
@@ -1060,8 +1060,8 @@ int expert_group_impl(ColiHipTensor *const *gates, ColiHipTensor *const *ups, Co
     int *row_exp = hi, *mt_exp = row_exp + total, *mt_row0 = mt_exp + T, *mt_rend = mt_row0 + T;
     int *mt_first = mt_rend + T;
     int *lead = mt_first + T;
-    int *counts = lead + T;
-    int *rp = counts + 4, *ri = rp + (red ? s_n + 1 : 0);
+    int *counts = lead + 1 + T;
+    int *rp = counts + 2, *ri = rp + (red ? s_n + 1 : 0);
     float *rwv = (float *)(ri + (red ? total : 0));
     int G = 0;
     for (int i = 0, r = 0, t = 0; i < count; i++) {
@@ -1072,14 +1072,13 @@ int expert_group_impl(ColiHipTensor *const *gates, ColiHipTensor *const *ups, Co
             mt_row0[t] = r + q;
             mt_rend[t] = r + rows[i];
             mt_first[t] = t0;
-            if (mmap::row_leads(t, t0)) lead[G++] = t;
+            if (mmap::row_leads(t, t0)) lead[1 + G++] = t;
         }
         r += rows[i];
     }
     counts[0] = total;
     counts[1] = T;
-    counts[2] = count;
-    counts[3] = G;
+    lead[0] = G;
     if (red) {
         std::memcpy(rp, red->row_ptr, (size_t)(s_n + 1) * 4);
         std::memcpy(ri, red->row_idx, (size_t)total * 4);
@@ -1096,7 +1095,7 @@ int expert_group_impl(ColiHipTensor *const *gates, ColiHipTensor *const *ups, Co
     plan.mt_rend = di + total + 2 * T;
     plan.mt_first = di + total + 3 * T;
     plan.lead = di + total + 4 * T;
-    plan.counts = di + total + 5 * T;
+    plan.counts = di + total + 5 * T + 1;
     // No copy engine in the call: the staging buffers are mapped host
     // memory. The activation quantisation reads x across PCIe and also stages
     // the metadata into device memory (every later kernel reads it there); the
@@ -1129,7 +1128,7 @@ int expert_group_impl(ColiHipTensor *const *gates, ColiHipTensor *const *ups, Co
         prof.mark(-1);
         if (phases) hipEventRecord(c->phase_ev[2], c->stream);
         if (red) {
-            const int *drp = plan.counts + 4, *dri = drp + s_n + 1;
+            const int *drp = plan.counts + 2, *dri = drp + s_n + 1;
             const float *drw = (const float *)(dri + total);
             prof.mark(COLI_HIP_K_COMBINE);
             launch_combine((float *)c->pin_y.d, s.y, drp, dri, drw, s_n, D, s.ys, c->stream);
@@ -1657,6 +1656,7 @@ int moe_forward_impl(const ColiHipExpertSet *set, const float *x_dev, int S, con
     // table layout in one buffer (the leading tiles last: the no-allocation
     // call does without them rather than be refused for them)
     int lead_max = arm == COLI_HIP_ARM_MFMA && row_groups(gg, gd, R, E, ga) ? mmap::row_lead_bound(R, std::min(E, R)) : 0;
+    auto lead_ints = [&]() -> size_t { return lead_max > 0 ? 1 + (size_t)lead_max : 0; };
     const size_t n_int = 4 + (size_t)E + (E + 1) + 3 * (size_t)R + 2 * (size_t)R + 4 * (size_t)tmax + table_work_ints(S, k, E);
     Scratch s{};
     int *p = nullptr;
@@ -1667,8 +1667,8 @@ int moe_forward_impl(const ColiHipExpertSet *set, const float *x_dev, int S, con
         size_t need = 0;
         if (!carve_rows(gg, gd, S, R, ga, nullptr, &need, &s)) return 0;
         const size_t tbl_off = need;
-        if (tbl_off + round_up((n_int + lead_max) * 4, 256) > COLI_HIP_FIXED_SCRATCH_BYTES) lead_max = 0;
-        need += round_up((n_int + lead_max) * 4, 256);
+        if (tbl_off + round_up((n_int + lead_ints()) * 4, 256) > COLI_HIP_FIXED_SCRATCH_BYTES) lead_max = 0;
+        need += round_up((n_int + lead_ints()) * 4, 256);
         if (need > COLI_HIP_FIXED_SCRATCH_BYTES) {
             std::fprintf(stderr,
                          "[HIP] moe_forward (no allocation): this call needs %zu bytes of scratch, more than the "
@@ -1679,7 +1679,7 @@ int moe_forward_impl(const ColiHipExpertSet *set, const float *x_dev, int S, con
         carve_rows(gg, gd, S, R, ga, c->fixed_scratch, &need, &s);
         p = (int *)(c->fixed_scratch + tbl_off);
     } else {
-        if (!reserve_rows(c, gg, gd, S, R, ga, &s) || !reserve(c, c->tbl, (n_int + lead_max) * 4)) return 0;
+        if (!reserve_rows(c, gg, gd, S, R, ga, &s) || !reserve(c, c->tbl, (n_int + lead_ints()) * 4)) return 0;
         p = (int *)c->tbl.p;
     }
     TableOut t{};

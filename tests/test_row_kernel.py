@@ -157,6 +157,10 @@ def test_row_kernel_layer(hip, orc, fmt, E, S, k, D, I):
     got = out.download(np.float32, (S, D))
     ok = (bad >= 0) & (bad < E)
     # the oracle takes ids in range: a skipped slot is its expert with weight 0, taken out of the order below
+    hdr = np.zeros(4, np.int32)
+    assert hip.lib.coli_hip_last_table(0, hip._ipt(hdr), None, None, None, None, 0, 0) == 1
+    counts = np.bincount(bad[ok], minlength=E)
+    assert list(hdr) == [ok.sum(), (-(-counts // MT)).sum(), (counts > 0).sum(), 0]   # the documented header
     ref = np.zeros((S, D), np.float32)
     y = np.zeros((E, S, D), np.float32)
     for e in range(E):
