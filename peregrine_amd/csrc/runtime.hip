@@ -16,6 +16,7 @@
 
 #include "../../include/peregrine_hip.h"
 #include "common.h"
+#include "host_rules.h"
 #include "mfma_map.h"
 
 using namespace phip;
@@ -1224,7 +1225,7 @@ int expert_group_impl(ColiHipTensor *const *gates, ColiHipTensor *const *ups, Co
     for (auto &e : c->phase_ev)
         if (phases && !e && hipEventCreateWithFlags(&e, hipEventDisableSystemFence) != hipSuccess) phases = false;
     for (int i = 0; n_chunk > 1 && i < n_chunk; i++) {
-        const int r0 = (int)((long)total * i / n_chunk), r1 = (int)((long)total * (i + 1) / n_chunk);
+        const int r0 = chunk_row(total, i, n_chunk, D), r1 = chunk_row(total, i + 1, n_chunk, D);
         std::memcpy((float *)c->pin_x.p + (size_t)r0 * D, x + (size_t)r0 * D, (size_t)(r1 - r0) * D * 4);
         launch_quant_rows(QuantArgs{x_dev + (size_t)r0 * D, D, r1 - r0, D, gg.Kp, s.xq + (size_t)r0 * s.xs, s.xs,
                                     s.sx + (size_t)r0 * s.sxs, s.sxs, epi_act(ga), (const uint4 *)opt.meta_src,
