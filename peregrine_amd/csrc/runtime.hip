@@ -28,9 +28,12 @@ using namespace phip;
 static __device__ __align__(256) uint8_t scratch[COLI_HIP_FIXED_SCRATCH_BYTES];
 // Per-tile arrival counters of the down GEMV's tail combine: zero at load,
 // and each dispatch leaves them zero again (the tile's last workgroup resets
-// its counter), so no clearing launch is needed. One stream per device uses
-// them; host code uses the address kept in Ctx::tail_ctr.
-static __device__ int tail_ctr[GEMV_TAIL_TILES];
+// its counter), so no clearing launch is needed. One set serves the dispatches
+// that use the context's scratch, the other those of the fixed scratch (the
+// no-allocation entry point): the two may run at the same time, a captured
+// no-allocation layer on a stream of its caller's. Host code uses the address
+// kept in Ctx::tail_ctr.
+static __device__ int tail_ctr[2 * GEMV_TAIL_TILES];
 // Per-unit arrival counters of the split-K GEMV, kept zero between
 // dispatches the same way (the unit's finishing workgroup resets its own).
 static __device__ int split_ctr[GEMV_SPLIT_UNITS];
@@ -110,7 +113,7 @@ struct Ctx {
     // device address of this device's copy of the fixed scratch array (the
     // no-allocation entry point), looked up at init with the device current
     uint8_t *fixed_scratch = nullptr;
-    int *tail_ctr = nullptr;   // this device's copy of tail_ctr[]
+    int *tail_ctr = nullptr;   // this device's copy of tail_ctr[]: the context's set, then the fixed scratch's
     int *split_ctr = nullptr;  // this device's copy of split_ctr[]
     // last device-resident table (for coli_hip_last_table)
     TableOut tbl_view{};
@@ -329,7 +332,7 @@ int check_waits(Ctx *c) {
     // clear the tail combine's tile counters too (the stream is idle here),
     // so a faulty dispatch cannot leave later ones a stale count
     if (c->tail_ctr) {
-        hipMemsetAsync(c->tail_ctr, 0, GEMV_TAIL_TILES * sizeof(int), c->stream);
+        hipMemsetAsync(c->tail_ctr, 0, 2 * GEMV_TAIL_TILES * sizeof(int), c->stream);
         if (c->split_ctr) hipMemsetAsync(c->split_ctr, 0, GEMV_SPLIT_UNITS * sizeof(int), c->stream);
         hipStreamSynchronize(c->stream);
     }
@@ -1768,7 +1771,7 @@ int moe_forward_impl(const ColiHipExpertSet *set, const float *x_dev, int S, con
     if (tail_c) {
         opt.tail_w = w_dev;
         opt.tail_out = out_dev;
-        opt.tail_ctr = c->tail_ctr;
+        opt.tail_ctr = c->tail_ctr + (fixed_scratch ? GEMV_TAIL_TILES : 0);
     }
     RowPlan plan{};
     if (one_token) {

@@ -3,6 +3,7 @@ against the allocating one (coli_hip_moe_forward_dev), through the C ABI:
 bit-identical on two calls in a row, the second smaller, on both arms; a call
 beyond the fixed scratch is refused. Collected last (it shares the device's
 fixed scratch array with nothing else, but runs after the other GPU tests)."""
+import ctypes as C
 import sys
 
 import numpy as np
@@ -113,6 +114,51 @@ def test_noalloc_replayed_from_a_graph(hip):
         got = bout.download(np.float32, (S, D))
         want = _run(hip, hip.moe_forward_dev, eset, x, ids, w, k, 32, -1)
         assert np.array_equal(got, want), rep
+
+
+def test_noalloc_one_token_beside_ordinary_calls(hip):
+    """A captured no-allocation layer of one token, replayed on a stream of its
+    own while ordinary one-token layers run on the device's: the two share no
+    scratch and no counter, so both stay right."""
+    say("no-alloc beside ordinary calls")
+    rt = hip.lib   # resolves the HIP runtime it links
+
+    def ck(rc):
+        assert rc == 0, rc
+    rng = np.random.default_rng(8)
+    E, D, I, k = 16, 5120, 1536, 8
+    _, eset = _layer(hip, rng, E, D, I)
+    case = []
+    for _ in range(2):
+        x = rng.standard_normal((1, D)).astype(np.float32)
+        ids, w = synth_route(rng, 1, E, k)
+        want = _run(hip, hip.moe_forward_dev, eset, x, ids, w, k, 32, -1)
+        case.append([hip.DeviceBuffer.from_array(a) for a in (x, ids, w)] + [hip.DeviceBuffer(D * 4), want])
+
+    def call(fn, c):
+        fn(eset, c[0].ptr, 1, c[1].ptr, c[2].ptr, k, c[3].ptr, 32, -1)
+    call(hip.moe_forward_dev_noalloc, case[0])
+    hip.pipe_sync(0)
+    dev, own, graph, ex = C.c_void_p(hip.stream_handle(0)), C.c_void_p(), C.c_void_p(), C.c_void_p()
+    ck(rt.hipStreamCreateWithFlags(C.byref(own), 1))
+    ck(rt.hipStreamBeginCapture(dev, 1))
+    call(hip.moe_forward_dev_noalloc, case[0])
+    ck(rt.hipStreamEndCapture(dev, C.byref(graph)))
+    ck(rt.hipGraphInstantiate(C.byref(ex), graph, None, None, C.c_size_t(0)))
+    for rep in range(50):
+        for c in case:
+            c[3].fill(D, 1, 5.0, 1.0, seed=rep)
+        hip.pipe_sync(0)
+        for _ in range(4):
+            ck(rt.hipGraphLaunch(ex, own))
+            call(hip.moe_forward_dev, case[1])
+        ck(rt.hipStreamSynchronize(own))
+        hip.pipe_sync(0)
+        for c in case:
+            assert np.array_equal(c[3].download(np.float32, (1, D)), c[4]), rep
+    ck(rt.hipGraphExecDestroy(ex))
+    ck(rt.hipGraphDestroy(graph))
+    ck(rt.hipStreamDestroy(own))
 
 
 def synth_route(rng, S, E, k):
