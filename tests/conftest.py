@@ -14,6 +14,17 @@ def pytest_configure(config):
 
 
 @pytest.fixture(scope="session")
+def host_rules(tmp_path_factory):
+    """The runtime's host decisions, built for the CPU."""
+    import ctypes
+    import subprocess
+    out = str(tmp_path_factory.mktemp("rules") / "libhost_rules.so")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC",
+                    os.path.join(ROOT, "tests", "native", "host_rules.cpp"), "-o", out], check=True)
+    return ctypes.CDLL(out)
+
+
+@pytest.fixture(scope="session")
 def orc():
     from oracle import oracle
     return oracle

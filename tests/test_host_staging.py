@@ -3,31 +3,17 @@ host copies the next. On the CPU: chunks cover x and start on whole cache
 lines, which the host and the GPU never share. On the GPU: calls with and
 without the reduce, on both arms, rows that do and do not end on a line,
 bit-identical to the oracle."""
-import ctypes
-import os
-import subprocess
-
 import numpy as np
 import pytest
 
 from peregrine_amd import qt, synth
 
-HERE = os.path.dirname(os.path.abspath(__file__))
-
-
-@pytest.fixture(scope="module")
-def rules(tmp_path_factory):
-    out = str(tmp_path_factory.mktemp("rules") / "libhost_rules.so")
-    subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", os.path.join(HERE, "native", "host_rules.cpp"),
-                    "-o", out], check=True)
-    return ctypes.CDLL(out)
-
 
 @pytest.mark.parametrize("D", [1, 8, 31, 36, 1000, 1001, 5120, 70001, 600000])
-def test_chunks_cover_x_on_whole_lines(rules, D):
+def test_chunks_cover_x_on_whole_lines(host_rules, D):
     for total in (1, 2, 33, 37, 192, 531, 4099):
         for n in range(2, 9):
-            at = [rules.chunk_row_c(total, i, n, D) for i in range(n + 1)]
+            at = [host_rules.chunk_row_c(total, i, n, D) for i in range(n + 1)]
             assert at[0] == 0 and at[n] == total and at == sorted(at)
             assert all(r * D * 4 % 128 == 0 for r in at[:n]), (total, n, at)
             assert all(b - a <= total / n + 33 for a, b in zip(at, at[1:])) or total < 32 * n

@@ -97,16 +97,11 @@ def test_row_kernel_offsets_reach_4gib(chk, rows_x, K):
         assert (bad == 0) == bool(chk.off32_ok_c(rows_x * K)) == (rows_x * K <= 1 << 32)
 
 
-def reaches_row_kernel(R, n, D, I):
-    """The dispatch rule (int4's, the narrower): rows per expert and items."""
-    return R >= (24 if D > 2016 else 64) * n and (R // 128 + n) * -(-(-(-I // 32) * 32) // 128) >= 256
-
-
 @pytest.mark.gpu
 @pytest.mark.parametrize("fmt", [qt.FMT_I4, qt.FMT_I8])
 @pytest.mark.parametrize("D,I", [(1000, 8130), (160, 8161), (96, 8192)])
 @pytest.mark.parametrize("rows", [[200, 1, 31, 95], [129, 128], [64, 97, 288]])
-def test_row_kernel_matches_oracle(hip, orc, fmt, D, I, rows):
+def test_row_kernel_matches_oracle(hip, orc, host_rules, fmt, D, I, rows):
     print("row kernel", fmt, D, I, rows, flush=True)
     rng = np.random.default_rng(D + I + fmt + len(rows))
     gpu, ora = [], []
@@ -114,7 +109,7 @@ def test_row_kernel_matches_oracle(hip, orc, fmt, D, I, rows):
         trip = synth.make_expert(rng, D, I, fmt, 32)
         gpu.append(hip.GpuExpert.upload_grouped(0, trip[0][:2], trip[1][:2], trip[2][:2], D, I, fmt, 32))
         ora.append(tuple(orc.Tensor(t[0], t[1], fmt, i, o, 32) for t, (o, i) in zip(trip, ((I, D), (I, D), (D, I)))))
-    assert reaches_row_kernel(sum(rows), len(rows), D, I)
+    assert host_rules.row_groups_c(D, I, int(fmt == qt.FMT_I4), 1, 1, sum(rows), len(rows), 0)   # as the runtime decides
     x = rng.standard_normal((sum(rows), D)).astype(np.float32)
     hip.set_act_group(0)
     hip.set_arm(0)
@@ -132,12 +127,12 @@ def test_row_kernel_matches_oracle(hip, orc, fmt, D, I, rows):
 @pytest.mark.gpu
 @pytest.mark.parametrize("fmt", [qt.FMT_I4, qt.FMT_I8])
 @pytest.mark.parametrize("E,S,k,D,I", [(5, 64, 3, 2048, 5440), (9, 300, 4, 2048, 1900), (3, 700, 3, 96, 1800)])
-def test_row_kernel_layer(hip, orc, fmt, E, S, k, D, I):
+def test_row_kernel_layer(hip, orc, host_rules, fmt, E, S, k, D, I):
     """The layer, whose leading tiles the device table lists (both table
     forms), with ids that skip an expert, repeat one and leave the range; at
     D = 2048 the rule's lower bound of 24 rows per expert holds too."""
     print("row layer", fmt, E, S, k, flush=True)
-    assert reaches_row_kernel(S * k, E, D, I)
+    assert host_rules.row_groups_c(D, I, int(fmt == qt.FMT_I4), 1, 1, S * k, E, 0)   # as the runtime decides
     rng = np.random.default_rng(E * S + fmt)
     gpu, ora = [], []
     for _ in range(E):
