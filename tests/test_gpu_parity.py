@@ -403,7 +403,7 @@ def test_moe_layer_matches_oracle(hip, orc, ga, arm):
     assert np.array_equal(t["tok_rows"].reshape(S, k), o["tok_rows"])
 
 
-@pytest.mark.parametrize("S,arm", [(1, -1), (1, 0), (6, 2), (6, -1)])
+@pytest.mark.parametrize("S,arm", [(1, -1), (1, 0), (6, 2), (6, -1), (6, 0)])
 @pytest.mark.parametrize("ga", [32, 0])
 def test_moe_layer_fused_router_matches_oracle(hip, orc, S, arm, ga):
     """Router fused with the x quantisation; one token on the GEMV arm runs

@@ -26,11 +26,11 @@ def hip():
     return h
 
 
-def _layer(hip, rng, E, D, I):
+def _layer(hip, rng, E, D, I, fmt=qt.FMT_I4G):
     gpu = []
     for _ in range(E):
-        trip = synth.make_expert(rng, D, I, qt.FMT_I4G, 32)
-        gpu.append(hip.GpuExpert.upload_grouped(0, trip[0][:2], trip[1][:2], trip[2][:2], D, I))
+        trip = synth.make_expert(rng, D, I, fmt, 32)
+        gpu.append(hip.GpuExpert.upload_grouped(0, trip[0][:2], trip[1][:2], trip[2][:2], D, I, fmt))
     return gpu, hip.ExpertSet(gpu)
 
 
@@ -114,6 +114,63 @@ def test_noalloc_replayed_from_a_graph(hip):
         got = bout.download(np.float32, (S, D))
         want = _run(hip, hip.moe_forward_dev, eset, x, ids, w, k, 32, -1)
         assert np.array_equal(got, want), rep
+
+
+@pytest.mark.parametrize("fmt", [qt.FMT_I4, qt.FMT_I8])
+@pytest.mark.parametrize("E,D,I,k,S,arm", [(9, 2048, 1900, 4, 300, -1), (9, 2048, 1900, 4, 3, 2), (9, 200, 1536, 4, 1, -1),
+                                           (5, 64, 4100, 2, 1, 2), (9, 2048, 1900, 4, 6, 0)])
+def test_noalloc_per_row_formats(hip, host_rules, fmt, E, D, I, k, S, arm):
+    """Per-row weights and activations: the 128-row GEMM, GEMVs that quantise
+    h themselves (and not, beyond 4096), one token with ids that repeat and
+    leave the range."""
+    say("no-alloc per row", fmt, E, D, I, k, S, arm)
+    assert bool(host_rules.row_groups_c(D, I, int(fmt == qt.FMT_I4), 1, 1, S * k, E, 0)) == (S == 300)
+    rng = np.random.default_rng(S + fmt)
+    _, eset = _layer(hip, rng, E, D, I, fmt)
+    for s in (S, max(1, S - 1)):
+        x = rng.standard_normal((s, D)).astype(np.float32)
+        ids = rng.integers(-1, E + 1, (s, k)).astype(np.int32)
+        w = rng.uniform(0.1, 1.0, (s, k)).astype(np.float32)
+        want = _run(hip, hip.moe_forward_dev, eset, x, ids, w, k, 0, arm)
+        got = _run(hip, hip.moe_forward_dev_noalloc, eset, x, ids, w, k, 0, arm)
+        assert np.array_equal(got, want) and np.abs(want).max() > 0, s
+
+
+def test_noalloc_per_row_at_the_scratch_limit(hip, host_rules):
+    """The most tokens that are accepted: the list of leading tiles (1287 words,
+    under 8 tokens' scratch) no longer fits there and the 32-row GEMM runs;
+    from 8 tokens fewer on it fits. The same bits on both sides."""
+    say("no-alloc per row limit")
+    rng = np.random.default_rng(64)
+    E, D, I = 512, 64, 64
+    _, eset = _layer(hip, rng, E, D, I, qt.FMT_I4)
+    top = 110000
+    x = rng.standard_normal((top, D)).astype(np.float32)
+    ids = rng.integers(0, E, (top, 1)).astype(np.int32)
+    w = rng.uniform(0.1, 1.0, (top, 1)).astype(np.float32)
+    bx, bi, bw = (hip.DeviceBuffer.from_array(a) for a in (x, ids, w))
+    out = hip.DeviceBuffer(top * D * 4)
+
+    def run(fn, S):
+        fn(eset, bx.ptr, S, bi.ptr, bw.ptr, 1, out.ptr, 0, 0)
+        hip.pipe_sync(0)
+        return out.download(np.float32, (S, D))
+
+    lo, hi = 90000, top   # accepted, refused
+    assert host_rules.row_groups_c(D, I, 1, 1, 1, lo, E, 0)
+    while hi - lo > 1:
+        S = (lo + hi) // 2
+        try:
+            hip.moe_forward_dev_noalloc(eset, bx.ptr, S, bi.ptr, bw.ptr, 1, out.ptr, 0, 0)
+            lo = S
+        except hip.HipError:
+            hi = S
+    assert lo > 90000
+    for S in (lo, lo - 4, lo - 7, lo - 8, lo - 9, lo - 60):
+        say("limit", S)
+        want = run(hip.moe_forward_dev, S)
+        got = run(hip.moe_forward_dev_noalloc, S)
+        assert np.array_equal(got, want) and np.abs(want).max() > 0, S
 
 
 def test_noalloc_one_token_beside_ordinary_calls(hip):
