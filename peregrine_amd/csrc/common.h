@@ -301,7 +301,7 @@ constexpr int ROUTE_MAX_E = 256;   // 4 logits per lane
 struct DotArgs {   // shared by the GEMV and MFMA arms
     const ExpertDesc *desc;
     RowPlan plan;
-    const int8_t *xq; int x_stride; const float *sx; int sx_stride;   // activations
+    const int8_t *xq; int x_stride, x_rows; const float *sx; int sx_stride;   // activations (x_rows: for the MFMA launches)
     float *out; int out_stride;                                         // h (gate/up) or y (down)
     int8_t *hq; int hq_stride; float *sh; int sh_stride;                // fused h quant (ACT_B32)
     int32_t *dots;                                                      // optional per-block dot dump
@@ -311,7 +311,6 @@ struct DotArgs {   // shared by the GEMV and MFMA arms
     int spin_limit;                                                     // GEMV: polls before a bounded wait gives up
     int *wait_failed;                                                   // GEMV: host-visible word, set to 1 when one does
     int w_reuse;                                                        // MFMA arm: M tiles re-read each expert's weights
-    int x_rows;                                                         // MFMA arm: rows of xq (its launch checks their bytes)
     int lead_bound;                                                     // > 0: per-row weights run mfma_row_kernel, G <= this
     RouteArgs route;                                                    // gate/up GEMV: logits != null -> fused router
     // down GEMV, one token (rows 0..n-1 in top-k order): the last workgroup
