@@ -81,7 +81,11 @@ int coli_hip_tensor_update(ColiHipTensor *tensor, const void *weights, const flo
 int coli_hip_expert_group(ColiHipTensor *const *gates, ColiHipTensor *const *ups, ColiHipTensor *const *downs,
                           const int *rows, int count, float *y, const float *x); /* coli_cuda_expert_group */
 /* tile_* are accepted and ignored (no WMMA fragment shapes on CDNA); arm_out
- * reports COLI_HIP_ARM_*. */
+ * reports COLI_HIP_ARM_*, the arm that this call ran. With no arm forced, a
+ * call with arm_out runs the GEMV where no expert has more than one row and the
+ * grouped GEMM otherwise; coli_hip_expert_group, coli_hip_expert_group_reduce
+ * and a call with arm_out = NULL run the GEMV for small batches too (the same
+ * bits, up to about twice as fast there), so arm_out does not tell their arm. */
 int coli_hip_expert_group_tiled(ColiHipTensor *const *gates, ColiHipTensor *const *ups,
                                 ColiHipTensor *const *downs, const int *rows, int count, float *y, const float *x,
                                 int tile_m, int tile_n, int tile_k, int *arm_out); /* coli_cuda_expert_group_tiled */
@@ -196,8 +200,9 @@ int coli_hip_moe_forward_dev(const ColiHipExpertSet *set, const float *x_dev, in
  * a fixed COLI_HIP_FIXED_SCRATCH_BYTES array per device, mapped at init; a
  * call needing more returns 0 with a message (about S * k <= 2300 rows at
  * D = 5120, I = 1536). Every call on a device shares that device's array and
- * leaves its contents behind: calls that overlap on one device (other host
- * threads, other streams) race. No profiling on this path. */
+ * leaves its contents behind: no-allocation calls that overlap on one device
+ * (other host threads, other streams) race with each other; with calls of the
+ * other entry points they share nothing. No profiling on this path. */
 #define COLI_HIP_FIXED_SCRATCH_BYTES (64 << 20)
 int coli_hip_moe_forward_dev_noalloc(const ColiHipExpertSet *set, const float *x_dev, int S, const int *ids_dev,
                                      const float *w_dev, int k, float *out_dev, int act_group, int arm);

@@ -52,6 +52,9 @@ bool row_groups(const Geom &gg, const Geom &gd, int R, int n, int ga) {
 // rows int4 33 / 44, 24 rows int8 45 / 45; 64 experts, D = 1024, I = 512, 48 rows
 // int4 30 / 35, 36 rows int8 36 / 35. Sharing does not turn it round: 1 expert,
 // D = 5120, 16 rows int4 37 / 90, int8 59 / 68; 4 experts, D = 2048, 32 rows 28 / 47.
+// So the bounds are on the safe side: 48 rows of the 160 experts lose to the
+// GEMM only with skewed popularity, and the crossings were not looked for by
+// activation mode (per-row activations gain most).
 template <class Geom>
 bool gemv_pays(const Geom &gg, const Geom &gd, int R) {
     const double bytes = (double)gg.Op * gg.Kp * (gg.w4 ? 1.0 : 2.0) + (double)gd.Op * gd.Kp * (gd.w4 ? 0.5 : 1.0);   // one expert's weights

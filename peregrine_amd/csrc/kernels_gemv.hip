@@ -675,7 +675,9 @@ __global__ __launch_bounds__(1024) void gemv_split_kernel(DotArgs a, MatGeom g, 
 // 14.2 us gate/up (14.4 with the ring) and 8.4-9.3 us down with the
 // quantisation (8.9 without, plus 3.4 us for its launch). 5 x 16 waves x blocks
 // for gate/up takes 20 us; 8 x 10, 11 x 5, 16 x 10 and down 6 x 8, 8 x 6, 3 x 8,
-// 2 x 12 measure within 1 us of 10 x 8 and 4 x 12.
+// 2 x 12 measure within 1 us of 10 x 8 and 4 x 12. All at these sizes, where
+// 10 x 8 is two whole rounds and 4 x 12 one; at others the waves past the last
+// block load it again for nothing.
 // ---------------------------------------------------------------------------
 constexpr int GEMV_ROW_MAXK = 4096;   // of the down projection: codes in LDS, 4 * HPER floats of h per thread
 constexpr int GEMV_ROW_MAXSUM = 65536;   // 16 x 8 x 127 x K stays below 2^31

@@ -85,7 +85,10 @@ __device__ __forceinline__ void table_one(const int *ids, int k, int E, const Ta
 // rows are short and many: bytes in flight, not the reduction, bound it.
 // Measured against quant_rows_kernel (4-byte loads, 1-byte stores): 14216 rows
 // of 1536 55 -> 20 us, 1777 rows of 5120 13.3 -> 10 us, 1800 rows of 736 9.5 ->
-// 4.9 us. Rows in host memory stay there: over PCIe the 4-byte loads are the
+// 4.9 us. One wave a row against four, back to back: 2.73 / 2.77 us at 256 rows
+// of 512 and 3.13 / 2.89 of 2048, 2.75 / 2.92 and 3.19 / 3.10 at 512, 2.75 /
+// 3.20 and 3.26 / 3.52 at 768, 5.1 / 11.6 and 13.9 / 15.3 at 8192: one wave from
+// 512 rows on. Rows in host memory stay there: over PCIe the 4-byte loads are the
 // faster ones (192 rows of 5120: 73 us against 94).
 template <int WPR>
 __global__ __launch_bounds__(256) void quant_rows_vec_kernel(QuantArgs a) {
